@@ -23,6 +23,7 @@ struct DevScalars {
     int inner_total;
     int pi_active;
     int pi_iter;
+    int inner_fail;             // a resident inner solve gave up waiting (dev_inner.hpp)
 };
 
 template <class T> __device__ __forceinline__ T clampv(T v, T lo, T hi) { return fmax(lo, fmin(v, hi)); }
@@ -400,7 +401,7 @@ constexpr int kRxLaneCols = 4;                      // columns of R per lane
 constexpr int kRxWaveCols = kWave * kRxLaneCols;    // columns of R per wave (one chunk)
 constexpr int kRxMaxRank = 256;
 
-inline int rx_chunks(int n) { return (n + kRxWaveCols - 1) / kRxWaveCols; }
+__host__ __device__ inline int rx_chunks(int n) { return (n + kRxWaveCols - 1) / kRxWaveCols; }
 
 // R is read once per pass: non-temporal loads keep it from displacing the
 // reused vectors in the caches.

@@ -24,6 +24,7 @@
 #include "../../include/pdhcg_amd.h"
 #include "dev_cones.hpp"
 #include "dev_sections.hpp"
+#include "dev_inner.hpp"
 #include "dev_kernels.hpp"
 #include "dev_timer.hpp"
 #include "host_scale.h"
@@ -595,6 +596,7 @@ template <class V, class X> class Solver final : public SolverBase {
     void read_scalars() {
         HIP_OK(hipMemcpyAsync(hs_, ds_, sizeof(DevScalars), hipMemcpyDeviceToHost, st_));
         HIP_OK(hipStreamSynchronize(st_));
+        if (hs_->inner_fail) fail("a resident inner solve waited too long for its workgroups");
     }
     int grid(long long n) const { return blocks_for(n); }
     // one thread per element, no cap (kernels without a grid reduction)
@@ -606,6 +608,8 @@ template <class V, class X> class Solver final : public SolverBase {
         cones_.project(v, var_rescale_, residual_warm, gate, st_);
     }
     void bb_prox(double tau, bool fuse_halpern, double w);
+    void init_inner_form();
+    void inner_launch(double tau, bool fuse_halpern, double w);
     void pdhg_step(bool fuse_halpern);
     void halpern(double w);
     void fixed_point_error();
@@ -702,6 +706,18 @@ template <class V, class X> class Solver final : public SolverBase {
     double *diag_h_ = nullptr;
     double cached_inv_tau_ = -1.0, inner_tol_ = 1e-3, inner_min_tol_ = 1e-9;
     int inner_limit_ = 1000;
+    // The inner solve as one launch of resident workgroups (dev_inner.hpp),
+    // for problems that fit the chip; kInnerLaunches enqueues its kernels one
+    // by one.
+    enum InnerForm { kInnerLaunches, kInnerLowRank, kInnerSparse };
+    InnerForm inner_form_ = kInnerLaunches;
+    int inner_groups_ = 0, inner_cols_ = 0;
+    size_t inner_lds_ = 0;
+    InnerExchange exchange_ = {};
+    // kInnerSparse: Q in row order, its rows cut into tasks
+    int *qrow_task_ = nullptr, *qtask_start_ = nullptr, *qci_ = nullptr;
+    V *qv_ = nullptr;
+    std::vector<int> row_task_;
     int host_inner_ = 0;  // +1 per outer iteration (reference pdhg_core_op.cu:762)
 
     // reductions and device scalars
@@ -872,6 +888,21 @@ template <class V, class X> void Solver<V, X>::upload(const ScaledProblem &sp) {
         } else {
             q_sparse_ = true;
             Q_ = upload_csr<V>(sp.Q);
+            // row order, cut into tasks, for the resident inner solve
+            if (qtype_ == PDHCG_SPARSE_Q && n_ <= kInnerSparseVars &&
+                sp.Q.nnz() <= kInnerSparseGroups * kInnerThreads * kInnerTask) {
+                std::vector<int> start;
+                row_task_.assign((size_t)n_ + 1, 0);
+                for (int i = 0; i < n_; ++i) {
+                    for (int e = sp.Q.rp[i]; e < sp.Q.rp[(size_t)i + 1]; e += kInnerTask) start.push_back(e);
+                    row_task_[(size_t)i + 1] = (int)start.size();
+                }
+                start.push_back(sp.Q.nnz());
+                qrow_task_ = dupload<int>(row_task_, row_task_.size());
+                qtask_start_ = dupload<int>(start, start.size());
+                qci_ = dupload<int>(sp.Q.ci, sp.Q.ci.size());
+                qv_ = dupload<V>(sp.Q.v, sp.Q.v.size());
+            }
         }
     }
     if (qtype_ == PDHCG_DIAG_Q) qdiag_ = dupload<X>(sp.qdiag, (size_t)n_);
@@ -1098,6 +1129,7 @@ template <class V, class X> void Solver<V, X>::init_inner(const ScaledProblem &s
     dirn_ = dzeros<X>(n_);
     if (has_cones_) snap_ = dzeros<X>(n_);
     precond_ = P_.diag_jacobi_precond && !has_psd_;
+    init_inner_form();
     if (!precond_) return;
     std::vector<double> dh((size_t)n_, 0.0);
     if (qtype_ == PDHCG_SPARSE_Q || qtype_ == PDHCG_LOW_RANK_PLUS_SPARSE_Q)
@@ -1133,6 +1165,117 @@ template <class V, class X> void Solver<V, X>::init_inner(const ScaledProblem &s
     minv_ = dzeros<X>(n_);
 }
 
+// Chooses the inner solve's form.  The resident forms need the whole
+// problem on the chip: a dense R of rank <= kInnerMaxRank in registers with
+// one column per thread of at most one workgroup per compute unit
+// (n <= 131 072), or a sparse Q whose x_p fits LDS and whose entries fit the
+// registers of kInnerSparseGroups workgroups.  Larger problems stream R or Q
+// from HBM or L2 in every body either way and keep the launches.  Measured on
+// MI355X in FP64, launches against resident, whole solves of 400 outer
+// iterations (milliseconds in the iteration): n = 600, rank 50: 80 -> 18;
+// n = 4000, rank 50: 136 -> 26; n = 20 000, rank 30: 99 -> 37; n = 100 000,
+// rank 50: 147 -> 52; n = 130 000, rank 50: 163 -> 56; sparse Q of 2000
+// variables (41 entries per row): 15-23 -> 5.5 us per body.
+template <class V, class X> void Solver<V, X>::init_inner_form() {
+    if (!bb_ || has_cones_ || n_ <= 0) return;
+    const bool plus = qtype_ == PDHCG_LOW_RANK_PLUS_SPARSE_Q;
+    int dev = 0, units = 0, coop = 0;
+    HIP_OK(hipGetDevice(&dev));
+    HIP_OK(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev));
+    HIP_OK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+    size_t rows = 0, total = 0, scalar = 0;
+    if ((qtype_ == PDHCG_LOW_RANK_Q || plus) && r_dense_ && !q_sparse_ && k_ > 0 && k_ <= kInnerMaxRank) {
+        const int groups = (n_ + kInnerCols - 1) / kInnerCols;
+        if (groups > kInnerPlainGroups && (!coop || groups > std::min(units, kInnerMaxGroups))) return;
+        inner_form_ = kInnerLowRank;
+        inner_groups_ = groups;
+        inner_cols_ = kInnerCols;
+        rows = (size_t)2 * (k_ + 1) * groups;
+        total = (size_t)2 * (k_ + 1);
+        scalar = (size_t)2 * groups;
+    } else if (qtype_ == PDHCG_SPARSE_Q && n_ <= kInnerSparseVars && (!q_sparse_ || qv_)) {
+        // at least 64 variables per workgroup, or as many workgroups as the
+        // entries of Q need for one task per thread
+        bool fits = false;
+        for (int groups = std::min(kInnerSparseGroups, (n_ + kWave - 1) / kWave); !fits && groups <= kInnerSparseGroups;
+             ++groups) {
+            inner_cols_ = (n_ + groups - 1) / groups;
+            inner_groups_ = (n_ + inner_cols_ - 1) / inner_cols_;
+            fits = true;
+            for (int g = 0; q_sparse_ && g < inner_groups_; ++g)
+                if (row_task_[std::min(n_, (g + 1) * inner_cols_)] - row_task_[g * inner_cols_] > kInnerThreads)
+                    fits = false;
+        }
+        if (!fits) return;
+        inner_form_ = kInnerSparse;
+        if (q_sparse_) {
+            inner_lds_ = (size_t)n_ * sizeof(double);
+            HIP_OK(hipFuncSetAttribute((const void *)inner_sparse_kernel<V, X, Acc>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)(kInnerSparseVars * sizeof(double))));
+        }
+        rows = (size_t)2 * n_;
+        scalar = (size_t)2 * inner_groups_ * kInnerWaves;
+    }
+    if (inner_form_ == kInnerLaunches) return;
+    exchange_.rows = dzeros<xword>(2 * rows);
+    exchange_.total = dzeros<xword>(2 * total);
+    exchange_.scalar = dzeros<xword>(2 * scalar);
+    exchange_.seq = dzeros<unsigned>(2);
+    int khz = 0;
+    HIP_OK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+    exchange_.wait = (long long)(kInnerWaitSeconds * 1e3 * std::max(khz, 1));
+}
+
+// One inner solve in its resident form.
+template <class V, class X> void Solver<V, X>::inner_launch(double tau, bool fuse_halpern, double w) {
+    InnerArgs<X> a{};
+    a.n = n_;
+    a.limit = inner_limit_;
+    a.halpern = fuse_halpern ? 1 : 0;
+    a.inv_tau = 1.0 / tau;
+    a.alpha0 = 1.0 / a.inv_tau;
+    a.tol = inner_tol_;
+    a.w = w;
+    a.rho = P_.reflection_coefficient;
+    a.x = x_;
+    a.xp = xp_;
+    a.xr = xr_;
+    a.x0 = x0_;
+    a.c = c_;
+    a.aty = aty_;
+    a.lb = lb_;
+    a.ub = ub_;
+    a.qdiag = qsdiag_;
+    a.m_inv = precond_ ? minv_ : nullptr;
+    a.m_diag = precond_ ? mdiag_ : nullptr;
+    a.ex = exchange_;
+    a.ds = ds_;
+    if (inner_form_ == kInnerSparse) {
+        hipLaunchKernelGGL((inner_sparse_kernel<V, X, Acc>), dim3(inner_groups_), dim3(kInnerThreads),
+                           inner_lds_, st_, a, inner_cols_, (const int *)qrow_task_, (const int *)qtask_start_,
+                           (const int *)qci_, (const V *)qv_);
+        HIP_OK(hipGetLastError());
+        return;
+    }
+    auto go = [&](auto kernel) {
+        const V *R = Rd_;
+        const double *dd = ddiag_, *de = ddense_;
+        void *args[] = {&a, &R, &k_, &dd, &de, &dkind_};
+        if (inner_groups_ > kInnerPlainGroups)
+            HIP_OK(hipLaunchCooperativeKernel((const void *)kernel, dim3(inner_groups_), dim3(kInnerThreads), args, 0,
+                                              st_));
+        else
+            HIP_OK(hipLaunchKernel((const void *)kernel, dim3(inner_groups_), dim3(kInnerThreads), args, 0, st_));
+    };
+    // rows of R per wave
+    if (k_ <= 8) go(inner_lowrank_kernel<V, X, 1>);
+    else if (k_ <= 16) go(inner_lowrank_kernel<V, X, 2>);
+    else if (k_ <= 32) go(inner_lowrank_kernel<V, X, 4>);
+    else if (k_ <= 56) go(inner_lowrank_kernel<V, X, 7>);
+    else go(inner_lowrank_kernel<V, X, 10>);
+}
+
 template <class V, class X> Solver<V, X>::~Solver() {
     if (st_) (void)hipStreamSynchronize(st_);
     delete eval_;
@@ -1150,6 +1293,7 @@ template <class V, class X> Solver<V, X>::~Solver() {
                     cu_fin_, lb_fin_, ub_fin_, con_rescale_, var_rescale_, x0_,     x_,           xp_,
                     xr_,     y0_,    y_,      yp_,     yr_,          aty_,        ax_,          dslack_,
                     dx_,     dy_,    qx_,     grad_,   dirn_,        mdiag_,      minv_,        diag_h_,
+                    exchange_.rows, exchange_.total, exchange_.scalar, exchange_.seq, qrow_task_, qtask_start_, qci_, qv_,
                     red_partials_, ds_, snap_, pgp_, dres_, aff_d_, acomp_, aproj_, apres_, amem_};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -1310,6 +1454,15 @@ template <class V, class X> void Solver<V, X>::bb_prox(double tau, bool fuse_hal
                            red());
         fold<1, 0>(nb, 0, TailTolScale{n_});
         cached_inv_tau_ = inv;
+    }
+    if (inner_form_ != kInnerLaunches) {
+        inner_launch(tau, fuse_halpern, w);
+        if (eval_) {  // the hand-over to FP64 counts inner solves that reached the limit
+            HIP_OK(hipMemcpyAsync(bb_poll_, &ds_->bb_iter, sizeof(int), hipMemcpyDeviceToHost, st_));
+            HIP_OK(hipStreamSynchronize(st_));
+            sat_run_ = (inner_limit_ > 1 && bb_poll_[0] >= inner_limit_) ? sat_run_ + 1 : 0;
+        }
+        return;
     }
     const X *mi = precond_ ? minv_ : nullptr;
     const X *md = precond_ ? mdiag_ : nullptr;
@@ -1703,6 +1856,7 @@ template <class V, class X> void Solver<V, X>::promote() {
             E.mdiag_ = dzeros<double>(n_);
             E.minv_ = dzeros<double>(n_);
         }
+        E.init_inner_form();
     }
     E.inner_tol_ = inner_tol_;
     E.inner_min_tol_ = inner_min_tol_;
