@@ -243,6 +243,12 @@ bool pack(const qp_problem_t *prob, const pdhg_parameters_t &P, Packed &k, const
             k.cones.push_back(Cone{(int)ac->type[c], ac->start_idx[c], ac->v_dim[c],
                                    ac->power_alpha ? ac->power_alpha[c] : 0.0});
         }
+    int widest = 0;
+    for (int c = 0; c < I.ncones - I.nlong; ++c)
+        if (k.cones[c].type == CONE_STANDARD_SOC || k.cones[c].type == CONE_ROTATED_SOC)
+            widest = std::max(widest, k.cones[c].vdim);
+    I.cone_lanes = widest <= 4 ? 4 : (widest <= 16 ? 16 : 64);
+    if ((long long)(I.ncones - I.nlong) * I.cone_lanes > 8LL * kBTSmall) I.cone_lanes = 0;
     // step size and primal weight (reference src/pdhg_core_op.cu:933-971)
     if (sp.A.nnz() == 0) I.step = 1.0;
     else {

@@ -50,6 +50,7 @@ struct Params {
 // One problem: sizes, pool offsets and scaled-problem scalars.
 struct Inst {
     int n, m, k, qkind, dkind, has_affine, ncones, cone0;
+    int cone_lanes;                // lanes per short SOC/RSOC cone (4, 16, 64), 0: one thread
     int nlong;                     // SOC/RSOC cones above kMaxThreadCone slots: the last nlong cones
     int a_rp, a_ci, at_rp, at_ci;  // int-pool offsets of [A;F] and its transpose
     int a_long, at_long;           // 1: a wavefront per row, 0: a thread per row
@@ -255,15 +256,45 @@ template <class T, int BT> struct Ctx {
         __syncthreads();
     }
 
+    // Second-order cones among the first nshort, L lanes per cone.
+    template <int L> __device__ void soc_groups(T *v, const T *d, double *warm, int nshort) const {
+        const int lane = threadIdx.x % L;
+        for (int c0 = 0; c0 < nshort; c0 += BT / L) {
+            const int c = c0 + (int)threadIdx.x / L;
+            Cone cn{CONE_EXPONENTIAL, 0, 0, 0.0};
+            if (c < nshort) cn = cones[c];
+            const bool live = cn.type == CONE_STANDARD_SOC || cn.type == CONE_ROTATED_SOC;
+            const int s = cn.start, k = cn.vdim;
+            const bool has = live && lane < k;
+            double p = has ? (double)v[s + lane] : 0.0, e = has ? (double)d[s + lane] : 1.0;
+            double a = live ? (double)v[s + k] : 0.0, b = live ? (double)v[s + k + 1] : 0.0;
+            const double ea = live ? (double)d[s + k] : 1.0, eb = live ? (double)d[s + k + 1] : 1.0;
+            soc_project_group<L>(live, p, e, lane, k, a, b, ea, eb, cn.type == CONE_ROTATED_SOC, warm + (live ? c : 0));
+            if (has) v[s + lane] = (T)p;
+            if (live && lane == 0) {
+                v[s + k] = (T)a;
+                v[s + k + 1] = (T)b;
+            }
+        }
+    }
+
     // Projection of the m-vector v onto the affine cones, scaling affd
-    // (reference src/cone_dispatch.cu:38-57 on the row space).
+    // (reference src/cone_dispatch.cu:38-57 on the row space).  Second-order
+    // cones take I.cone_lanes lanes each (soc_project_group): with one thread
+    // per cone a portfolio's pass took about 30 us more, in the bisection of
+    // its one cone of 12 to 52 slots (256 portfolios: 783 -> 698 ms).  With more cones than eight rounds of the workgroup's groups hold
+    // (cone_lanes 0) a thread per cone is the faster form.
     __device__ __noinline__ void project_affine(T *v, double *warm) const {
         const T *d = mv(wAFD);
         const int nshort = I.ncones - I.nlong;
+        if (I.cone_lanes == 4) soc_groups<4>(v, d, warm, nshort);
+        else if (I.cone_lanes == 16) soc_groups<16>(v, d, warm, nshort);
+        else if (I.cone_lanes == 64) soc_groups<64>(v, d, warm, nshort);
         for (int c = threadIdx.x; c < nshort; c += BT) {
             const Cone cn = cones[c];
             const int s = cn.start;
             if (cn.type == CONE_STANDARD_SOC || cn.type == CONE_ROTATED_SOC) {
+                if (I.cone_lanes) continue;
                 double pv[kMaxThreadCone + 2];
                 for (int q = 0; q < cn.vdim + 2; ++q) pv[q] = v[s + q];
                 if constexpr (std::is_same<T, double>::value) {

@@ -173,6 +173,7 @@ class DevConeSet {
   public:
     bool psd = false, power = false;
     ConeList rsoc, soc, expc, powc;
+    SocClasses rsoc_cls = {}, soc_cls = {};      // lane classes of the rsoc and soc lists
     ConeList lrsoc, lsoc;                        // SOC/RSOC blocks above kMaxThreadCone vector slots
     ConeList powall;                             // every power block, for the primal violation
     SectionList sec;                             // blocks with fixed slots (any non-PSD type)
@@ -249,6 +250,27 @@ class DevConeSet {
             lists[li].start.push_back(st);
             lists[li].vdim.push_back(vd);
             lists[li].alpha.push_back(t == CONE_POWER && b->power_alpha ? b->power_alpha[k] : 0.0);
+        }
+        // SOC and RSOC blocks in the order of their lane classes
+        for (int li = 0; li < 2; ++li) {
+            HostList &h = lists[li], sorted;
+            SocClasses &cls = li == 0 ? rsoc_cls : soc_cls;
+            int groups = 0;
+            for (int c = 0; c < kSocClasses; ++c) {
+                cls.first[c] = (int)sorted.start.size();
+                cls.group[c] = groups;
+                for (size_t i = 0; i < h.start.size(); ++i) {
+                    if (soc_class_of(h.vdim[i]) != c) continue;
+                    sorted.start.push_back(h.start[i]);
+                    sorted.vdim.push_back(h.vdim[i]);
+                    sorted.alpha.push_back(h.alpha[i]);
+                }
+                const long long lanes = ((long long)sorted.start.size() - cls.first[c]) * (4LL << c);
+                groups += (int)((lanes + kBlock - 1) / kBlock);
+            }
+            cls.first[kSocClasses] = (int)sorted.start.size();
+            cls.group[kSocClasses] = groups;
+            h = std::move(sorted);
         }
         ConeList *dst[6] = {&rsoc, &soc, &expc, &powc, &lrsoc, &lsoc};
         for (int li = 0; li < 6; ++li) {
@@ -355,17 +377,17 @@ class DevConeSet {
             HIP_OK(hipEventRecord(join_, side_));
         }
         if (rsoc.count)
-            hipLaunchKernelGGL((cone_project_kernel<X, CONE_ROTATED_SOC>), blocks(rsoc.count), dim3(kBlock), 0, st, v,
-                               d, rsoc, rw, gate);
+            hipLaunchKernelGGL((soc_project_kernel<X, true>), dim3(rsoc_cls.group[kSocClasses]), dim3(kBlock), 0, st, v, d,
+                               (const X *)nullptr, 0.0, rsoc, rsoc_cls, rw, gate);
         if (soc.count)
-            hipLaunchKernelGGL((cone_project_kernel<X, CONE_STANDARD_SOC>), blocks(soc.count), dim3(kBlock), 0, st, v,
-                               d, soc, rw, gate);
+            hipLaunchKernelGGL((soc_project_kernel<X, false>), dim3(soc_cls.group[kSocClasses]), dim3(kBlock), 0, st, v, d,
+                               (const X *)nullptr, 0.0, soc, soc_cls, rw, gate);
         if (expc.count)
             hipLaunchKernelGGL((cone_project_kernel<X, CONE_EXPONENTIAL>), blocks(expc.count), dim3(kBlock), 0, st, v,
-                               d, expc, rw, gate);
+                               d, expc, gate);
         if (powc.count)
             hipLaunchKernelGGL((cone_project_kernel<X, CONE_POWER>), blocks(powc.count), dim3(kBlock), 0, st, v, d,
-                               powc, rw, gate);
+                               powc, gate);
         if (lrsoc.count)
             hipLaunchKernelGGL((soc_long_project_kernel<X, true>), dim3(lrsoc.count), dim3(kBlock), 0, st, v, d,
                                (const X *)nullptr, 0.0, lrsoc, rw, gate);
@@ -386,11 +408,11 @@ class DevConeSet {
     // metric diag(1 + tau q) (PSD blocks excluded; they take the BB path).
     template <class X> void project_diag_q(X *v, const double *d, const X *q, double tau, hipStream_t st) const {
         if (rsoc.count)
-            hipLaunchKernelGGL((cone_project_diag_q_kernel<X, CONE_ROTATED_SOC>), blocks(rsoc.count), dim3(kBlock), 0,
-                               st, v, d, q, tau, rsoc);
+            hipLaunchKernelGGL((soc_project_kernel<X, true>), dim3(rsoc_cls.group[kSocClasses]), dim3(kBlock), 0, st, v, d,
+                               q, tau, rsoc, rsoc_cls, 0, (const int *)nullptr);
         if (soc.count)
-            hipLaunchKernelGGL((cone_project_diag_q_kernel<X, CONE_STANDARD_SOC>), blocks(soc.count), dim3(kBlock), 0,
-                               st, v, d, q, tau, soc);
+            hipLaunchKernelGGL((soc_project_kernel<X, false>), dim3(soc_cls.group[kSocClasses]), dim3(kBlock), 0, st, v, d,
+                               q, tau, soc, soc_cls, 0, (const int *)nullptr);
         if (expc.count)
             hipLaunchKernelGGL((cone_project_diag_q_kernel<X, CONE_EXPONENTIAL>), blocks(expc.count), dim3(kBlock), 0,
                                st, v, d, q, tau, expc);
