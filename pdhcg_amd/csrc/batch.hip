@@ -59,12 +59,12 @@ __global__ void widen_iterates_kernel(const Inst *insts, const float *s32, doubl
     const int mv[] = {wY0, wY, wYP, wYR, wAX, wDY, wPRES, wPSL, wAPR, wAMEM};
     for (int w : nv)
         for (int i = threadIdx.x; i < I.n; i += blockDim.x) {
-            const long long o = I.vec + (long long)w * I.n + i;
+            const long long o = I.vec + (long long)w * I.pn + i;
             s64[o] = (double)s32[o];
         }
     for (int w : mv)
         for (int i = threadIdx.x; i < I.m; i += blockDim.x) {
-            const long long o = I.vec + (long long)kNVec * I.n + (long long)w * I.m + i;
+            const long long o = I.vec + (long long)kNVec * I.pn + (long long)w * I.pm + i;
             s64[o] = (double)s32[o];
         }
 }
@@ -142,6 +142,18 @@ const char *unsupported(const qp_problem_t *p) {
     return nullptr;
 }
 
+// Chunk table of a product (dev_batch.hpp spmv) appended to `out`: the first
+// row that starts in each chunk or later, then `rows`.
+void chunk_table(const std::vector<int> &rp, int rows, int nnz, std::vector<int> &out) {
+    const int chunks = chunk_count(nnz);
+    int r = 0;
+    for (int c = 0; c < chunks; ++c) {
+        while (r < rows && rp[r] < (long long)c * kChunk) ++r;
+        out.push_back(r);
+    }
+    out.push_back(rows);
+}
+
 // Scales and packs one problem; returns false (with *why set) for an
 // objective the batch does not handle.
 bool pack(const qp_problem_t *prob, const pdhg_parameters_t &P, Packed &k, const char **why) {
@@ -162,6 +174,8 @@ bool pack(const qp_problem_t *prob, const pdhg_parameters_t &P, Packed &k, const
     Inst &I = k.inst;
     I.n = n;
     I.m = m;
+    I.pn = padded4(n);
+    I.pm = padded4(m);
     I.k = 0;
     I.cbr = sp.cbr;
     I.ovr = sp.ovr;
@@ -185,22 +199,36 @@ bool pack(const qp_problem_t *prob, const pdhg_parameters_t &P, Packed &k, const
             for (int i = 0; i < n; ++i)
                 for (int q = sp.Q.rp[i]; q < sp.Q.rp[(size_t)i + 1]; ++q) qd[i] += sp.Q.v[q];
     }
-    // pools: [A rp | A ci | At rp | At ci] and [A v | At v | R | D]
+    // pools: [A rp | A ci | At rp | At ci | chunk tables] and [A v | At v | R | D].
+    // An A whose dense form (8 bytes a position) is smaller than its two CSR
+    // forms (24 bytes an entry) is stored dense: a portfolio's products with it
+    // took 57 000 and 59 000 of 275 000 cycles a pass in CSR.
     const HostCSR At = transpose(sp.A);
-    I.a_rp = 0;
-    I.a_ci = m + 1;
-    I.at_rp = I.a_ci + sp.A.nnz();
-    I.at_ci = I.at_rp + n + 1;
-    k.ai.insert(k.ai.end(), sp.A.rp.begin(), sp.A.rp.end());
-    k.ai.insert(k.ai.end(), sp.A.ci.begin(), sp.A.ci.end());
-    k.ai.insert(k.ai.end(), At.rp.begin(), At.rp.end());
-    k.ai.insert(k.ai.end(), At.ci.begin(), At.ci.end());
-    I.a_long = sp.A.nnz() >= 16LL * std::max(m, 1);
-    I.at_long = At.nnz() >= 16LL * std::max(n, 1);
-    I.a_v = 0;
-    I.at_v = sp.A.nnz();
-    k.av.insert(k.av.end(), sp.A.v.begin(), sp.A.v.end());
-    k.av.insert(k.av.end(), At.v.begin(), At.v.end());
+    I.a_nnz = sp.A.nnz();
+    I.a_dense = m <= kMaxRank && 3LL * I.a_nnz >= (long long)m * n;
+    I.a_v = I.at_v = 0;
+    if (I.a_dense) {
+        k.av.assign((size_t)m * I.pn, 0.0);
+        for (int i = 0; i < m; ++i)
+            for (int q = sp.A.rp[i]; q < sp.A.rp[(size_t)i + 1]; ++q) k.av[(size_t)i * I.pn + sp.A.ci[q]] += sp.A.v[q];
+    } else {
+        I.a_rp = 0;
+        I.a_ci = m + 1;
+        I.at_rp = I.a_ci + I.a_nnz;
+        I.at_ci = I.at_rp + n + 1;
+        k.ai.insert(k.ai.end(), sp.A.rp.begin(), sp.A.rp.end());
+        k.ai.insert(k.ai.end(), sp.A.ci.begin(), sp.A.ci.end());
+        k.ai.insert(k.ai.end(), At.rp.begin(), At.rp.end());
+        k.ai.insert(k.ai.end(), At.ci.begin(), At.ci.end());
+        I.a_chunk = (int)k.ai.size();
+        chunk_table(sp.A.rp, m, I.a_nnz, k.ai);
+        I.at_chunk = (int)k.ai.size();
+        chunk_table(At.rp, n, I.a_nnz, k.ai);
+        I.at_v = I.a_nnz;
+        k.av.insert(k.av.end(), sp.A.v.begin(), sp.A.v.end());
+        k.av.insert(k.av.end(), At.v.begin(), At.v.end());
+    }
+    k.av.resize((k.av.size() + 3) & ~(size_t)3, 0.0);  // R's rows are read in aligned pairs
     I.rdense = (long long)k.av.size();
     if (I.qkind == kQLowRank) {
         std::vector<double> Rd((size_t)r * n, 0.0);
@@ -221,11 +249,15 @@ bool pack(const qp_problem_t *prob, const pdhg_parameters_t &P, Packed &k, const
             }
             dh[i] += acc;
         }
-        k.av.insert(k.av.end(), Rd.begin(), Rd.end());
+        for (int j = 0; j < r; ++j) {
+            k.av.insert(k.av.end(), Rd.begin() + (size_t)j * n, Rd.begin() + (size_t)(j + 1) * n);
+            k.av.resize(k.av.size() + (size_t)(I.pn - n), 0.0);
+        }
     }
     I.dmat = (long long)k.av.size();
     if (sp.dkind == MiddleKind::Diag) k.av.insert(k.av.end(), sp.ddiag.begin(), sp.ddiag.end());
     if (sp.dkind == MiddleKind::Dense) k.av.insert(k.av.end(), sp.ddense.begin(), sp.ddense.end());
+    k.av.resize((k.av.size() + 3) & ~(size_t)3, 0.0);
     // affine cones on the rows
     const cone_blocks_t *ac = sp.affine_cones;
     I.ncones = (ac && m > 0) ? ac->num_cones : 0;
@@ -259,8 +291,8 @@ bool pack(const qp_problem_t *prob, const pdhg_parameters_t &P, Packed &k, const
     // the slab (FP64), starting point projected onto the box
     k.slab.assign((size_t)slab_size(n, m), 0.0);
     k.wslab.assign((size_t)wslab_size(I.k, I.ncones), 0.0);
-    auto N = [&](int w) { return k.slab.data() + (size_t)w * n; };
-    auto M = [&](int w) { return k.slab.data() + (size_t)kNVec * n + (size_t)w * m; };
+    auto N = [&](int w) { return k.slab.data() + (size_t)w * I.pn; };
+    auto M = [&](int w) { return k.slab.data() + (size_t)kNVec * I.pn + (size_t)w * I.pm; };
     for (int i = 0; i < n; ++i) {
         N(vC)[i] = sp.c[i];
         N(vLB)[i] = sp.lb[i];
@@ -341,13 +373,10 @@ struct ShapeKey {
         return std::tie(mixed, count, n, m, nnz) < std::tie(o.mixed, o.count, o.n, o.m, o.nnz);
     }
 };
-struct ShapeChoice {
-    int threads, row_len;
-};
 std::mutex g_shape_mu;
-std::map<ShapeKey, ShapeChoice> g_shapes;
+std::map<ShapeKey, int> g_shapes;  // threads per problem
 
-bool lookup_shape(const ShapeKey &k, ShapeChoice &out) {
+bool lookup_shape(const ShapeKey &k, int &out) {
     std::lock_guard<std::mutex> lock(g_shape_mu);
     auto it = g_shapes.find(k);
     if (it == g_shapes.end()) return false;
@@ -355,9 +384,9 @@ bool lookup_shape(const ShapeKey &k, ShapeChoice &out) {
     return true;
 }
 
-void store_shape(const ShapeKey &k, const ShapeChoice &c) {
+void store_shape(const ShapeKey &k, int threads) {
     std::lock_guard<std::mutex> lock(g_shape_mu);
-    g_shapes[k] = c;
+    g_shapes[k] = threads;
 }
 
 }  // namespace
@@ -437,6 +466,8 @@ extern "C" int pdhcg_solve_batch(const qp_problem_t *const *problems, int count,
             I.a_ci += io;
             I.at_rp += io;
             I.at_ci += io;
+            I.a_chunk += io;
+            I.at_chunk += io;
             I.a_v += vo;
             I.at_v += vo;
             I.rdense += vo;
@@ -451,17 +482,23 @@ extern "C" int pdhcg_solve_batch(const qp_problem_t *const *problems, int count,
             std::copy(q.wslab.begin(), q.wslab.end(), wslabs.get() + woff[b]);
             // every offset the kernel derives from I stays inside this
             // problem's share of the pools (a failure is a packing bug)
-            const long long nnz = (long long)q.inst.at_rp - q.inst.a_ci;
-            const int *rp = ipool.get() + I.a_rp, *trp = ipool.get() + I.at_rp;
-            bool ok = I.a_ci == I.a_rp + I.m + 1 && (long long)I.at_rp == I.a_ci + nnz &&
-                      I.at_ci == I.at_rp + I.n + 1 && I.at_ci + nnz <= ioff[b + 1] && rp[0] == 0 &&
-                      rp[I.m] == nnz && trp[0] == 0 && trp[I.n] == nnz && I.at_v == I.a_v + nnz &&
-                      I.rdense == I.at_v + nnz && I.dmat >= I.rdense && I.dmat <= voff[b + 1] &&
-                      I.vec + slab_size(I.n, I.m) <= soff[b + 1] && I.wvec + wslab_size(I.k, I.ncones) <= woff[b + 1] &&
-                      I.cone0 + I.ncones <= coff[b + 1];
-            for (long long e = 0; ok && e < nnz; ++e) {
-                const int c = ipool[(size_t)I.a_ci + e], r = ipool[(size_t)I.at_ci + e];
-                ok = c >= 0 && c < I.n && r >= 0 && r < I.m;
+            const long long nnz = I.a_nnz;
+            bool ok = I.rdense % 4 == 0 && I.vec % 4 == 0 && I.dmat >= I.rdense + (long long)I.k * I.pn &&
+                      I.dmat <= voff[b + 1] && I.vec + slab_size(I.n, I.m) <= soff[b + 1] &&
+                      I.wvec + wslab_size(I.k, I.ncones) <= woff[b + 1] && I.cone0 + I.ncones <= coff[b + 1];
+            if (I.a_dense) {
+                ok = ok && I.m <= kMaxRank && I.a_v % 4 == 0 && I.rdense >= I.a_v + (long long)I.m * I.pn;
+            } else {
+                const int *rp = ipool.get() + I.a_rp, *trp = ipool.get() + I.at_rp;
+                ok = ok && I.a_ci == I.a_rp + I.m + 1 && (long long)I.at_rp == I.a_ci + nnz &&
+                     I.at_ci == I.at_rp + I.n + 1 && I.a_chunk == I.at_ci + nnz &&
+                     I.at_chunk == I.a_chunk + chunk_count(I.a_nnz) + 1 &&
+                     I.at_chunk + chunk_count(I.a_nnz) + 1 <= ioff[b + 1] && rp[0] == 0 && rp[I.m] == nnz &&
+                     trp[0] == 0 && trp[I.n] == nnz && I.at_v == I.a_v + nnz && I.rdense >= I.at_v + nnz;
+                for (long long e = 0; ok && e < nnz; ++e) {
+                    const int c = ipool[(size_t)I.a_ci + e], r = ipool[(size_t)I.at_ci + e];
+                    ok = c >= 0 && c < I.n && r >= 0 && r < I.m;
+                }
             }
             for (int c = 0; ok && c < I.ncones; ++c) {
                 const Cone &cn = cones[(size_t)I.cone0 + c];
@@ -580,73 +617,60 @@ extern "C" int pdhcg_solve_batch(const qp_problem_t *const *problems, int count,
                 }
             }
         };
+        // dynamic LDS: one workgroup of 512 threads per compute unit, or two of 256
+        int lds_max = 0, device = 0;
+        HIP_OK(hipGetDevice(&device));
+        HIP_OK(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+        const int lds_large = std::max(0, lds_max - kStaticLds), lds_small = std::max(0, lds_max / 2 - kStaticLds);
+        auto allow_lds = [](auto kernel, int bytes) {
+            HIP_OK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+        };
+        allow_lds(batch_solve_kernel<double, kBT>, lds_large);
+        allow_lds(batch_solve_kernel<double, kBTSmall>, lds_small);
+        allow_lds(batch_solve_kernel<float, kBT>, lds_large);
+        allow_lds(batch_solve_kernel<float, kBTSmall>, lds_small);
         // launches of the main phase's kernel at either workgroup size
         auto launch32 = [&](int bt, int budget) {
             if (bt == kBTSmall)
-                hipLaunchKernelGGL((batch_solve_kernel<float, kBTSmall>), dim3(B), dim3(kBTSmall), 0, st, d_params,
+                hipLaunchKernelGGL((batch_solve_kernel<float, kBTSmall>), dim3(B), dim3(kBTSmall), lds_small, st, d_params,
                                    d_insts, d_ipool, (const float *)d_vpool32, (const double *)d_vpool, d_slabs32,
-                                   d_wslabs, d_cones, d_states, d_out, budget);
+                                   d_wslabs, d_cones, d_states, d_out, budget, lds_small);
             else
-                hipLaunchKernelGGL((batch_solve_kernel<float, kBT>), dim3(B), dim3(kBT), 0, st, d_params, d_insts,
+                hipLaunchKernelGGL((batch_solve_kernel<float, kBT>), dim3(B), dim3(kBT), lds_large, st, d_params, d_insts,
                                    d_ipool, (const float *)d_vpool32, (const double *)d_vpool, d_slabs32, d_wslabs,
-                                   d_cones, d_states, d_out, budget);
+                                   d_cones, d_states, d_out, budget, lds_large);
         };
         auto launch64 = [&](int bt, int budget) {
             if (bt == kBTSmall)
-                hipLaunchKernelGGL((batch_solve_kernel<double, kBTSmall>), dim3(B), dim3(kBTSmall), 0, st, d_params,
+                hipLaunchKernelGGL((batch_solve_kernel<double, kBTSmall>), dim3(B), dim3(kBTSmall), lds_small, st, d_params,
                                    d_insts, d_ipool, (const double *)d_vpool, (const double *)d_vpool, d_slabs,
-                                   d_wslabs, d_cones, d_states, d_out, budget);
+                                   d_wslabs, d_cones, d_states, d_out, budget, lds_small);
             else
-                hipLaunchKernelGGL((batch_solve_kernel<double, kBT>), dim3(B), dim3(kBT), 0, st, d_params, d_insts,
+                hipLaunchKernelGGL((batch_solve_kernel<double, kBT>), dim3(B), dim3(kBT), lds_large, st, d_params, d_insts,
                                    d_ipool, (const double *)d_vpool, (const double *)d_vpool, d_slabs, d_wslabs,
-                                   d_cones, d_states, d_out, budget);
+                                   d_cones, d_states, d_out, budget, lds_large);
         };
-        // Launch-shape autotuning.  Each candidate runs the same short probe
-        // from the same saved state (loop states, slabs and FP64 slabs are
-        // copied device-to-device and restored after each), and the batch
-        // runs with the fastest, kept only when 5% faster than the default:
-        //   threads per problem, 512 or 256;
-        //   then, when some problem's A or A' has rows of 4 to 63 entries on
-        //   average (either form could win), the row length from which a
-        //   product takes a wavefront per row instead of a thread per row:
-        //   16 (default), 4 or 64.
-        // PDHCG_BATCH_THREADS=256|512 and PDHCG_BATCH_ROWS=4|16|64 pin them.
-        // The choice is kept per process for the batch's shape (precision,
-        // problem count, total n, m and nnz(A)), so a family solved again
-        // (cold, warm, at another tolerance) is not probed again.
-        int bt = kBT, row_len = 16;
+        // Launch-shape autotuning: 512 and 256 threads per problem run the same
+        // short probe from the same saved state (loop states, slabs and FP64
+        // slabs are copied device-to-device and restored after each), and the
+        // batch runs with 256 when that is 5% faster.  PDHCG_BATCH_THREADS
+        // pins it.  The choice is kept per process for the batch's shape
+        // (precision, problem count, total n, m and nnz(A)), so a family solved
+        // again (cold, warm, at another tolerance) is not probed again.
+        int bt = kBT;
         const char *et = std::getenv("PDHCG_BATCH_THREADS");
-        const char *er = std::getenv("PDHCG_BATCH_ROWS");
         if (et) bt = std::atoi(et) == kBTSmall ? kBTSmall : kBT;
-        if (er && (std::atoi(er) == 4 || std::atoi(er) == 64)) row_len = std::atoi(er);
-        auto set_rows = [&](int len) {  // the per-problem row forms for a threshold, on the device
-            for (Inst &I : insts) {
-                const long long nnz = (long long)I.at_rp - I.a_ci;
-                I.a_long = nnz >= (long long)len * std::max(I.m, 1);
-                I.at_long = nnz >= (long long)len * std::max(I.n, 1);
-            }
-            HIP_OK(hipMemcpyAsync(d_insts, insts.data(), (size_t)B * sizeof(Inst), hipMemcpyHostToDevice, st));
-        };
-        bool ambiguous = false;
-        for (const Inst &I : insts) {
-            const long long nnz = (long long)I.at_rp - I.a_ci;
-            for (int rows : {I.m, I.n})
-                if (rows > 0 && nnz >= 4LL * rows && nnz < 64LL * rows) ambiguous = true;
-        }
         long long tot_n = 0, tot_m = 0, tot_nnz = 0;
         for (const Inst &I : insts) {
             tot_n += I.n;
             tot_m += I.m;
-            tot_nnz += (long long)I.at_rp - I.a_ci;
+            tot_nnz += I.a_nnz;
         }
         const ShapeKey key{mixed ? 1 : 0, B, tot_n, tot_m, tot_nnz};
-        ShapeChoice known{};
+        int known = 0;
         const bool have = lookup_shape(key, known);
-        if (have && !et) bt = known.threads;
-        if (have && !er) row_len = known.row_len;
-        if (row_len != 16) set_rows(row_len);
-        const bool tune_bt = !et && !have && window > 1, tune_rows = !er && !have && ambiguous && window > 1;
-        if (tune_bt || tune_rows) {
+        if (have && !et) bt = known;
+        if (!et && !have && window > 1) {
             const int probe = std::min(window, 12);
             const size_t sbytes = (size_t)soff[B] * (mixed ? sizeof(float) : sizeof(double));
             void *slab_src = mixed ? (void *)d_slabs32 : (void *)d_slabs;
@@ -688,33 +712,14 @@ extern "C" int pdhcg_solve_batch(const qp_problem_t *const *problems, int count,
                 return ms;
             };
             copy_all(true);
-            if (tune_bt) {
-                const float m512 = timed(kBT), m256 = timed(kBTSmall);
-                bt = m256 < 0.95f * m512 ? kBTSmall : kBT;
-                if (P.verbose >= 1)
-                    std::fprintf(stderr,
-                                 "[batch] threads per problem: %d (probe of %d passes: 512 -> %.1f ms, 256 -> %.1f ms)\n",
-                                 bt, probe, m512, m256);
-            }
-            if (tune_rows) {
-                const int lens[3] = {16, 4, 64};
-                float ms[3];
-                for (int c = 0; c < 3; ++c) {
-                    set_rows(lens[c]);
-                    ms[c] = timed(bt);
-                }
-                int best = 0;
-                for (int c = 1; c < 3; ++c)
-                    if (ms[c] < 0.95f * ms[0] && ms[c] < ms[best]) best = c;
-                row_len = lens[best];
-                set_rows(row_len);
-                if (P.verbose >= 1)
-                    std::fprintf(stderr,
-                                 "[batch] wavefront rows from %d entries (probe: 16 -> %.1f ms, 4 -> %.1f ms, 64 -> %.1f ms)\n",
-                                 row_len, ms[0], ms[1], ms[2]);
-            }
+            const float m512 = timed(kBT), m256 = timed(kBTSmall);
+            bt = m256 < 0.95f * m512 ? kBTSmall : kBT;
+            if (P.verbose >= 1)
+                std::fprintf(stderr,
+                             "[batch] threads per problem: %d (probe of %d passes: 512 -> %.1f ms, 256 -> %.1f ms)\n",
+                             bt, probe, m512, m256);
             HIP_OK(hipStreamSynchronize(st));
-            if (!et && !er) store_shape(key, ShapeChoice{bt, row_len});  // only fully probed choices
+            store_shape(key, bt);
         }
         if (mixed) {
             run_phase([&] { launch32(bt, window); }, "FP32", INT_MAX);
@@ -753,8 +758,8 @@ extern "C" int pdhcg_solve_batch(const qp_problem_t *const *problems, int count,
             const ScaledProblem &sp = pk[b].sp;
             const Out &o = out[b];
             const double *V = slabs.get() + I.vec;
-            const double *xp = V + (size_t)vXP * I.n, *aty = V + (size_t)vATY * I.n, *qx = V + (size_t)vQX * I.n;
-            const double *yp = V + (size_t)kNVec * I.n + (size_t)wYP * I.m;
+            const double *xp = V + (size_t)vXP * I.pn, *aty = V + (size_t)vATY * I.pn, *qx = V + (size_t)vQX * I.pn;
+            const double *yp = V + (size_t)kNVec * I.pn + (size_t)wYP * I.pm;
             pdhcg_result_t *r = ccalloc<pdhcg_result_t>(1);
             r->primal_solution = cmalloc<double>(I.n);
             r->dual_solution = cmalloc<double>(I.m);

@@ -1,5 +1,5 @@
 // Batched solve: many independent problems in one persistent launch, one
-// 256-thread workgroup per problem running the whole restarted Halpern PDHG
+// workgroup per problem running the whole restarted Halpern PDHG
 // loop of reference src/solver.cu:121-169 on the device (evaluation cadence,
 // KKT residuals, restarts with the PID primal weight, the BB inner solve,
 // affine cones, termination).  The arithmetic follows the single-problem
@@ -13,10 +13,19 @@
 // waves per SIMD with 512 threads per problem (fully inlined at 256 threads
 // it needed 294 registers and ran one problem per CU).
 //
-// Supported per problem: box bounds, rows [A; F] in CSR, objective of type
-// LP, diagonal Q, or dense low rank R'DR (k <= 64) plus a diagonal part, and
-// affine cones (SOC / RSOC up to 64 vector slots, exponential, power) on the
-// rows.  Variable cones and off-diagonal sparse Q are handled by the
+// What bounds it: with 256 problems or more running, the matrices and vectors
+// of every problem stream through the memory-side cache in every pass, about
+// 35 GB/s per compute unit; alone, the chain of dependent passes behind
+// barriers.  So as many rows of R as fit stay in LDS for the whole launch, a
+// mostly full A is stored dense (one copy without indices), the rest is read in
+// 16-byte pieces with eight or more in flight per lane, and an inner body is
+// two passes over the columns.  Measured on whole batches of 256 in FP64, start
+// of this form against it: portfolios of 50 to 2000 assets 698 -> 352 ms,
+// 2000-variable instances with rank 50 and power-law rows 740 -> 465 ms.
+//
+// Supported per problem: box bounds, rows [A; F], objective of type LP,
+// diagonal Q, or dense low rank R'DR (k <= 256) plus a diagonal part, and
+// affine cones (SOC / RSOC, exponential, power) on the rows.  Variable cones and off-diagonal sparse Q are handled by the
 // single-problem solver only.
 #pragma once
 
@@ -34,7 +43,8 @@ namespace batch {
 // parameter BT, a compile-time constant.
 constexpr int kBT = 512, kBTSmall = 256;
 constexpr int kBW = kBT / kWave;  // waves of the largest workgroup (reduction slots)
-constexpr int kMaxRank = 256;  // low-rank terms up to this rank (R x, u live in the slab)
+constexpr int kStaticLds = 1024;  // bound on the kernel's static LDS (reductions)
+constexpr int kMaxRank = 256;  // low-rank terms up to this rank (R x and D R x live in LDS)
 
 enum QKind { kQNone = 0, kQDiag = 1, kQLowRank = 2 };
 
@@ -50,14 +60,16 @@ struct Params {
 // One problem: sizes, pool offsets and scaled-problem scalars.
 struct Inst {
     int n, m, k, qkind, dkind, has_affine, ncones, cone0;
+    int pn, pm;                    // n and m rounded up to 4: pitch of the slab's vectors and of R's rows
     int cone_lanes;                // lanes per short SOC/RSOC cone (4, 16, 64), 0: one thread
     int nlong;                     // SOC/RSOC cones above kMaxThreadCone slots: the last nlong cones
     int a_rp, a_ci, at_rp, at_ci;  // int-pool offsets of [A;F] and its transpose
-    int a_long, at_long;           // 1: a wavefront per row, 0: a thread per row
+    int a_dense;                   // 1: A is stored dense (m x pn row-major at a_v), no CSR and no transpose
+    int a_nnz, a_chunk, at_chunk;  // entries of A; int-pool offsets of the products' chunk tables
     long long a_v, at_v;           // value-pool offsets of the matrix values
     long long vec;                 // slab offset of the problem's n- and m-vectors
     long long wvec;                // FP64 slab offset of its k-vectors and per-cone values
-    long long rdense, dmat;        // value-pool offsets of R (k x n row-major) and D
+    long long rdense, dmat;        // value-pool offsets of R (k x pn row-major, zero padded) and D
     double cbr, ovr, obj_const, obj_norm, bound_norm, step, pw0, nonconvexity;
 };
 
@@ -78,11 +90,21 @@ struct Out {
 enum NVec { vC, vLB, vUB, vVR, vQD, vDH, vX0, vX, vXP, vXR, vATY, vDS, vGR, vDIR, vQX, vPB, vDX, vMD, vMI, vLBF, vUBF,
             kNVec };
 enum MVec { wG, wCL, wCU, wCLF, wCUF, wCR, wY0, wY, wYP, wYR, wAX, wDY, wPRES, wPSL, wAPR, wAMEM, wAFD, kMVec };
-constexpr int kKVec = 2;      // rx, rx buffer
+constexpr int kKVec = 0;      // the k-vectors live in LDS
 constexpr int kConeVals = 3;  // projection warm start, residual warm start, complementarity
 
-inline long long slab_size(int n, int m) { return (long long)kNVec * n + (long long)kMVec * m; }
+__host__ __device__ inline int padded4(int n) { return (n + 3) & ~3; }
+inline long long slab_size(int n, int m) {
+    return (long long)kNVec * padded4(n) + (long long)kMVec * padded4(m);
+}
 inline long long wslab_size(int k, int ncones) { return (long long)kKVec * k + (long long)kConeVals * ncones; }
+
+// Chunks of kChunk entries in which a product streams its matrix, at least one.
+constexpr int kChunk = 4096;
+__host__ __device__ inline int chunk_count(int nnz) {
+    const int c = (nnz + kChunk - 1) / kChunk;
+    return c > 0 ? c : 1;
+}
 
 __device__ inline int print_frequency(int it) {
     int step = 10;
@@ -100,7 +122,7 @@ __device__ inline double clampd(double v, double lo, double hi) { return fmax(lo
 template <int BT> struct Red {
     double *lds;  // 2 * kBW doubles
     __device__ double sum(double v) const {
-        v = wave_sum(v);
+        v = wave_total(v);
         const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
         if (lane == 0) lds[w] = v;
         __syncthreads();
@@ -135,45 +157,155 @@ template <int BT> struct Red {
     }
 };
 
-// y = M x for a CSR matrix of `rows` rows.  With one workgroup per problem
-// and two waves per SIMD there is little occupancy to hide memory latency,
-// so each lane keeps four independent partial sums (four loads in flight)
-// and adds them in a fixed order.
+// Two adjacent elements in global memory (aligned: every pitch is a multiple
+// of four elements).  The address space is named because the pointers come
+// from a structure in memory: the compiler would use flat accesses, which
+// also wait for LDS.
+template <class T> struct Pair {
+    typedef T type __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(1))) type global;
+    typedef __attribute__((address_space(1))) T scalar;
+};
+typedef const __attribute__((address_space(1))) int *GlobalInt;
+template <class T> __device__ __forceinline__ typename Pair<T>::type load_pair(const T *p) {
+    return *(const typename Pair<T>::global *)p;
+}
+template <class T> __device__ __forceinline__ void store_pair(T *p, T a, T b) {
+    typename Pair<T>::type v = {a, b};
+    *(typename Pair<T>::global *)p = v;
+}
+
+// Dynamic LDS: D R x and R x (kMaxRank doubles each), then elements of the
+// storage type: the vector a product is taken of (when it fits), a chunk of a
+// sparse product and the first rows of R (Ctx::stage_room, room).
+extern __shared__ __align__(16) double batch_lds[];
+__device__ __forceinline__ double *lds_u() { return batch_lds; }
+__device__ __forceinline__ double *lds_rx() { return batch_lds + kMaxRank; }
+template <class T> __device__ __forceinline__ T *lds_room() { return reinterpret_cast<T *>(batch_lds + 2 * kMaxRank); }
+template <class T> __device__ __forceinline__ typename Pair<T>::type load_pair_lds(int i) {
+    return *reinterpret_cast<const typename Pair<T>::type *>(lds_room<T>() + i);
+}
+template <class T> __device__ __forceinline__ void store_pair_lds(int i, T a, T b) {
+    typename Pair<T>::type v = {a, b};
+    *reinterpret_cast<typename Pair<T>::type *>(lds_room<T>() + i) = v;
+}
+
+// y = M x for a CSR matrix of `rows` rows and `nnz` entries.  With one
+// workgroup per problem and two waves per SIMD there is little occupancy to
+// hide memory latency, and a row per lane group is a chain of three dependent
+// loads per few rows: 150 us for 1000 power-law rows of 20 entries on average,
+// 25 us for 1300 rows of 24.  So the entries are streamed in chunks of kChunk
+// whatever the rows: column and value of every entry of the next two chunks are
+// in flight while this one's products, in LDS, are summed by row (chunk_row[c]:
+// first row that starts in chunk c or later; a row that continues from the
+// chunk before is added to).  Rows longer than 32 entries per lane of the
+// chunk's groups take the whole wavefront.  x is copied to LDS first when it
+// fits (prod_at: its room): a gather from the caches takes the address unit a
+// cycle per lane, 4000 a chunk.  Measured in a batch of 256: 1000 power-law
+// rows of 20 entries 150 -> 29 us, their transpose 36 -> 21 us.
 template <class T, int BT>
-__device__ inline void spmv(const int *rp, const int *ci, const T *v, const T *x, T *y, int rows,
-                            int wave_rows) {
-    if (wave_rows) {
-        const int lane = threadIdx.x % kWave;
-        for (int r = threadIdx.x / kWave; r < rows; r += BT / kWave) {
-            T s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-            const int end = rp[r + 1];
-            int e = rp[r] + lane;
-            for (; e + 3 * kWave < end; e += 4 * kWave) {
-                s0 += v[e] * x[ci[e]];
-                s1 += v[e + kWave] * x[ci[e + kWave]];
-                s2 += v[e + 2 * kWave] * x[ci[e + 2 * kWave]];
-                s3 += v[e + 3 * kWave] * x[ci[e + 3 * kWave]];
-            }
-            for (; e < end; e += kWave) s0 += v[e] * x[ci[e]];
-            const T s = wave_sum((s0 + s1) + (s2 + s3));
-            if (lane == 0) y[r] = s;
+__device__ __noinline__ void spmv(const int *rp_, const int *ci_, const T *v_, const int *chunk_row_, const T *x_,
+                                  T *y_, int rows, int nnz, int cols, int prod_at) {
+    const auto rp = (GlobalInt)rp_, ci = (GlobalInt)ci_, chunk_row = (GlobalInt)chunk_row_;
+    const auto v = (const typename Pair<T>::scalar *)v_, x = (const typename Pair<T>::scalar *)x_;
+    const auto y = (typename Pair<T>::scalar *)y_;
+    constexpr int E = kChunk / BT, W = BT / kWave;
+    T *prod = lds_room<T>() + prod_at;
+    const T *xs = lds_room<T>();
+    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    const int chunks = chunk_count(nnz);
+    struct Entries {
+        int col[E];
+        T val[E];
+    } even, odd;
+    auto fetch = [&](Entries &b, int c) {
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int e = c * kChunk + tid + q * BT;
+            b.col[q] = e < nnz ? ci[e] : -1;
+            b.val[q] = e < nnz ? v[e] : T(0);
         }
-    } else {
-        for (int r = threadIdx.x; r < rows; r += BT) {
-            T s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-            const int end = rp[r + 1];
-            int e = rp[r];
-            for (; e + 3 < end; e += 4) {
-                s0 += v[e] * x[ci[e]];
-                s1 += v[e + 1] * x[ci[e + 1]];
-                s2 += v[e + 2] * x[ci[e + 2]];
-                s3 += v[e + 3] * x[ci[e + 3]];
-            }
-            for (; e < end; ++e) s0 += v[e] * x[ci[e]];
-            y[r] = (s0 + s1) + (s2 + s3);
+    };
+    // sum of prod[i], i = from, from + step, ... < to, four loads in flight
+    auto strided = [&](int from, int to, int step) {
+        T acc[4] = {T(0), T(0), T(0), T(0)};
+        for (int i = from; i < to; i += 4 * step) {
+            T p[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) p[q] = prod[min(i + q * step, kChunk - 1)];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (i + q * step < to) acc[q] += p[q];
         }
+        return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    };
+    int r0 = 0, r1 = chunk_row[1];
+    auto process = [&](Entries &b, int c) {
+        T g[E];
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            g[q] = T(0);
+            if (b.col[q] >= 0) g[q] = prod_at ? xs[b.col[q]] : x[b.col[q]];
+        }
+#pragma unroll
+        for (int q = 0; q < E; ++q)
+            if (b.col[q] >= 0) prod[tid + q * BT] = b.val[q] * g[q];
+        // lanes per row that starts here, and this group's first row
+        const int count = r1 - r0;
+        int lanes = kWave;
+        while (lanes > 1 && lanes * count > BT) lanes >>= 1;
+        const int per = BT / lanes, sub = tid & (lanes - 1), first = r0 + tid / lanes;
+        int s = first < r1 ? rp[first] : 0, e = first < r1 ? rp[first + 1] : 0;
+        const int next = chunk_row[min(c + 2, chunks)];
+        const int cont_end = c > 0 ? rp[r0] : 0;  // end of the row before r0
+        if (c + 2 < chunks) fetch(b, c + 2);
+        __syncthreads();
+        const int base = c * kChunk, top = min(base + kChunk, nnz);
+        for (int k0 = r0; k0 < r1; k0 += per) {
+            const int r = k0 + tid / lanes;
+            if (k0 != r0) {
+                s = r < r1 ? rp[r] : 0;
+                e = r < r1 ? rp[r + 1] : 0;
+            }
+            const int end = min(e, top);
+            const bool mine = r < r1 && end - s <= 32 * lanes;
+            double t = mine ? (double)strided(s - base + sub, end - base, lanes) : 0.0;
+            if (lanes >= 2) t += dpp_move<kDppXor1>(t);
+            if (lanes >= 4) t += dpp_move<kDppXor2>(t);
+            if (lanes >= 8) t += dpp_move<kDppHalfMirror>(t);
+            if (lanes >= 16) t += dpp_move<kDppMirror>(t);
+            if (lanes >= 32) t = fold16(t, t);
+            if (lanes >= 64) t = fold32(t, t);
+            if (mine && sub == 0) y[r] = (T)t;
+            unsigned long long mask = __ballot(sub == 0 && r < r1 && !mine);
+            for (; mask; mask &= mask - 1) {  // long rows: the whole wavefront
+                const int src = __ffsll((long long)mask) - 1;
+                const int row = __shfl(r, src, kWave), from = __shfl(s, src, kWave) - base;
+                const double w = wave_total((double)strided(from + lane, __shfl(end, src, kWave) - base, kWave));
+                if (lane == 0) y[row] = (T)w;
+            }
+        }
+        if (cont_end > base && wave == W - 1) {
+            const double t = wave_total((double)strided(lane, min(cont_end, top) - base, kWave));
+            if (lane == 0) y[r0 - 1] = (T)((double)y[r0 - 1] + t);
+        }
+        r0 = r1;
+        r1 = next;
+        __syncthreads();
+    };
+    fetch(even, 0);
+    if (chunks > 1) fetch(odd, 1);
+    if (prod_at) {
+        for (int p = tid; p < padded4(cols) / 2; p += BT) {
+            const auto w = load_pair(x_ + 2 * p);
+            store_pair_lds<T>(2 * p, w[0], w[1]);
+        }
+        __syncthreads();
     }
-    __syncthreads();
+    for (int c = 0; c < chunks; c += 2) {
+        process(even, c);
+        if (c + 1 < chunks) process(odd, c + 1);
+    }
 }
 
 // Everything one problem's loop needs, as device pointers.  T is the
@@ -183,23 +315,200 @@ __device__ inline void spmv(const int *rp, const int *ci, const T *v, const T *x
 template <class T, int BT> struct Ctx {
     const Params *P;
     Inst I;
-    const int *arp, *aci, *atrp, *atci;
+    const int *arp, *aci, *atrp, *atci, *ach, *atch;
     const T *av, *atv, *R;
     const double *D;
     T *V;       // n- and m-vectors of the slab
-    double *W;  // k-vectors and per-cone values (FP64)
+    double *W;  // per-cone values (FP64)
     const Cone *cones;
     Red<BT> red;
-    __device__ T *nv(int which) const { return V + (long long)which * I.n; }
-    __device__ T *mv(int which) const { return V + (long long)kNVec * I.n + (long long)which * I.m; }
-    __device__ double *kv(int which) const { return W + (long long)which * I.k; }
+    // LDS: room for the vector of a product (at 0; 0: not staged), then a chunk
+    // of a sparse product, then (offset `room`) the first `resident` rows of
+    // R, which are loaded once per launch
+    int stage_room, room, resident;
+    __device__ T *nv(int which) const { return V + (long long)which * I.pn; }
+    __device__ T *mv(int which) const { return V + (long long)kNVec * I.pn + (long long)which * I.pm; }
     __device__ double *cv(int which) const { return W + (long long)kKVec * I.k + (long long)which * I.ncones; }
-    __device__ void A(const T *x, T *y) const { spmv<T, BT>(arp, aci, av, x, y, I.m, I.a_long); }
-    __device__ void At(const T *y, T *x) const { spmv<T, BT>(atrp, atci, atv, y, x, I.n, I.at_long); }
+    // Products with A and A'.  A dense A (factor models: a few full rows) is
+    // read once per product without indices, by the passes of a dense R.
+    __device__ void A(const T *x, T *y) const {
+        if (I.a_dense) dense_rows(x, y);
+        else spmv<T, BT>(arp, aci, av, ach, x, y, I.m, I.a_nnz, I.n, stage_room);
+    }
+    __device__ void At(const T *y, T *x) const {
+        if (I.a_dense) dense_columns(y, x);
+        else spmv<T, BT>(atrp, atci, atv, atch, y, x, I.n, I.a_nnz, I.m, stage_room);
+    }
+    __device__ __noinline__ void dense_rows(const T *x, T *y) const {
+        stage(x);
+        __syncthreads();
+        auto put = [&](int r, double v) { y[r] = (T)v; };
+        if (stage_room) all_rows(av, I.m, 0, [&](int i) { return load_pair_lds<T>(i); }, put);
+        else all_rows(av, I.m, 0, [&](int i) { return load_pair(x + i); }, put);
+        __syncthreads();
+    }
+    __device__ __noinline__ void dense_columns(const T *y, T *x) const {
+        for (int i = threadIdx.x; i < I.m; i += BT) lds_rx()[i] = (double)y[i];
+        __syncthreads();
+        for (int p = threadIdx.x; p < I.pn / 2; p += BT) {
+            T v[2];
+            columns(av, I.m, 0, lds_rx(), p, v);
+            store_pair(x + 2 * p, v[0], v[1]);
+        }
+        __syncthreads();
+    }
+
+    // Sums of U rows of R times x over the wave; the lanes take pairs of
+    // columns, four per row in flight.  row(a, i), x(i): the pair at column i.
+    template <int U, class Row, class Vec> __device__ __forceinline__ void row_sums(Row row, Vec x, double (&out)[U]) const {
+        typedef typename Pair<T>::type P2;
+        const int half = I.pn / 2, lane = threadIdx.x % kWave;
+        T s[U][2];
+#pragma unroll
+        for (int a = 0; a < U; ++a) s[a][0] = s[a][1] = T(0);
+        for (int p = lane; p < half; p += 4 * kWave) {
+            P2 v[U][4], xv[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const bool in = p + q * kWave < half;
+                xv[q] = P2(T(0));
+                if (in) xv[q] = x(2 * (p + q * kWave));
+#pragma unroll
+                for (int a = 0; a < U; ++a) {
+                    v[a][q] = P2(T(0));
+                    if (in) v[a][q] = row(a, 2 * (p + q * kWave));
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int a = 0; a < U; ++a) {
+                    s[a][0] += v[a][q][0] * xv[q][0];
+                    s[a][1] += v[a][q][1] * xv[q][1];
+                }
+        }
+#pragma unroll
+        for (int a = 0; a < U; ++a) out[a] = wave_total((double)s[a][0] + (double)s[a][1]);
+    }
+    // put(r, row r of M times x) in lane 0, for the rows [0, k) of a dense
+    // k x pn M whose first `res` rows are the resident ones in LDS; x(i) as in
+    // row_sums (staged x: written before a barrier).
+    template <class Vec, class Put>
+    __device__ __forceinline__ void all_rows(const T *M, int k, int res, Vec x, Put put) const {
+        constexpr int W = BT / kWave;
+        const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+        for (int r = res + wave; r < k; r += 2 * W) {
+            const T *r0 = M + (long long)r * I.pn, *r1 = r0 + (long long)W * I.pn;
+            if (r + W < k) {
+                double v[2];
+                row_sums<2>([&](int a, int i) { return load_pair((a ? r1 : r0) + i); }, x, v);
+                if (lane == 0) {
+                    put(r, v[0]);
+                    put(r + W, v[1]);
+                }
+            } else {
+                double v[1];
+                row_sums<1>([&](int, int i) { return load_pair(r0 + i); }, x, v);
+                if (lane == 0) put(r, v[0]);
+            }
+        }
+        for (int r = wave; r < res; r += W) {
+            const int r0 = room + r * I.pn;
+            double v[1];
+            row_sums<1>([&](int, int i) { return load_pair_lds<T>(r0 + i); }, x, v);
+            if (lane == 0) put(r, v[0]);
+        }
+    }
+    // u = D R x (in LDS); ends with a barrier.
+    template <class Vec> __device__ __forceinline__ void low_rank_rows(Vec x) const {
+        const int k = I.k;
+        all_rows(R, k, resident, x, [&](int r, double v) {
+            if (I.dkind == 2) lds_rx()[r] = v;
+            else lds_u()[r] = I.dkind == 1 ? v * D[r] : v;
+        });
+        __syncthreads();
+        if (I.dkind == 2) {  // the symmetric part of a dense D from its upper triangle (reference src/pdhg_core_op.cu:272-303)
+            for (int i = threadIdx.x; i < k; i += BT) {
+                double a = 0.0;
+                for (int j = 0; j < k; ++j) {
+                    const int lo = i < j ? i : j, hi = i < j ? j : i;
+                    a += D[(long long)lo * k + hi] * lds_rx()[j];
+                }
+                lds_u()[i] = a;
+            }
+            __syncthreads();
+        }
+    }
+    __device__ __forceinline__ void low_rank_u(const T *x) const {
+        if (stage_room) low_rank_rows([&](int i) { return load_pair_lds<T>(i); });
+        else low_rank_rows([&](int i) { return load_pair(x + i); });
+    }
+    // Columns 2 p and 2 p + 1 of R'u.
+    __device__ __forceinline__ void low_rank_columns(int p, T (&out)[2]) const {
+        columns(R, I.k, resident, lds_u(), p, out);
+    }
+    // Columns 2 p and 2 p + 1 of M'u for the M of all_rows and u in LDS.  The
+    // first eight rows outside LDS are in flight while the resident ones are
+    // added.
+    __device__ __forceinline__ void columns(const T *M, int k, int resident, const double *u, int p, T (&out)[2]) const {
+        typedef typename Pair<T>::type P2;
+        constexpr int U = 8;
+        const int pn = I.pn, lcol = room + 2 * p;
+        const T *col = M + 2 * p;
+        T s0 = T(0), s1 = T(0);
+        int r = resident;
+        P2 g[U];
+#pragma unroll
+        for (int a = 0; a < U; ++a) {
+            g[a] = P2(T(0));
+            if (r + a < k) g[a] = load_pair(col + (long long)(r + a) * pn);
+        }
+        for (int j = 0; j < resident; j += 4) {
+            P2 v[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                v[a] = P2(T(0));
+                if (j + a < resident) v[a] = load_pair_lds<T>(lcol + (j + a) * pn);
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const T uj = j + a < resident ? (T)u[j + a] : T(0);
+                s0 += v[a][0] * uj;
+                s1 += v[a][1] * uj;
+            }
+        }
+        while (r < k) {
+            P2 nx[U];
+#pragma unroll
+            for (int a = 0; a < U; ++a) {
+                nx[a] = P2(T(0));
+                if (r + U + a < k) nx[a] = load_pair(col + (long long)(r + U + a) * pn);
+            }
+#pragma unroll
+            for (int a = 0; a < U; ++a) {
+                const T uj = r + a < k ? (T)u[r + a] : T(0);
+                s0 += g[a][0] * uj;
+                s1 += g[a][1] * uj;
+            }
+#pragma unroll
+            for (int a = 0; a < U; ++a) g[a] = nx[a];
+            r += U;
+        }
+        out[0] = s0;
+        out[1] = s1;
+    }
+    // Copies x into LDS (when the product's vector is staged); a barrier must follow.
+    __device__ __forceinline__ void stage(const T *x) const {
+        if (!stage_room) return;
+        for (int p = threadIdx.x; p < I.pn / 2; p += BT) {
+            const auto v = load_pair(x + 2 * p);
+            store_pair_lds<T>(2 * p, v[0], v[1]);
+        }
+    }
 
     // qx = Q x (reference src/pdhg_core_op.cu:305-413): diagonal part plus R'DR x
     __device__ __noinline__ void obj_product(const T *x, T *qx) const {
-        const int n = I.n, k = I.k;
+        const int n = I.n;
         if (I.qkind == kQNone) return;
         const T *qd = nv(vQD);
         if (I.qkind == kQDiag) {
@@ -207,51 +516,14 @@ template <class T, int BT> struct Ctx {
             __syncthreads();
             return;
         }
-        double *rx = kv(0), *rb = kv(1);
-        const int lane = threadIdx.x % kWave;
-        for (int r = threadIdx.x / kWave; r < k; r += BT / kWave) {
-            const T *row = R + (long long)r * n;
-            T s0 = 0, s1 = 0, s2 = 0, s3 = 0;  // four loads in flight, fixed order
-            int j = lane;
-            for (; j + 3 * kWave < n; j += 4 * kWave) {
-                s0 += row[j] * x[j];
-                s1 += row[j + kWave] * x[j + kWave];
-                s2 += row[j + 2 * kWave] * x[j + 2 * kWave];
-                s3 += row[j + 3 * kWave] * x[j + 3 * kWave];
-            }
-            for (; j < n; j += kWave) s0 += row[j] * x[j];
-            const double s = (double)wave_sum((s0 + s1) + (s2 + s3));
-            if (lane == 0) rx[r] = s;
-        }
+        stage(x);
         __syncthreads();
-        // u = D rx: diagonal, or the symmetric part of a dense D from its
-        // upper triangle (reference src/pdhg_core_op.cu:272-303)
-        if (I.dkind == 1) {
-            for (int r = threadIdx.x; r < k; r += BT) rb[r] = rx[r] * D[r];
-        } else if (I.dkind == 2) {
-            for (int i = threadIdx.x; i < k; i += BT) {
-                double a = 0.0;
-                for (int j = 0; j < k; ++j) {
-                    const int lo = i < j ? i : j, hi = i < j ? j : i;
-                    a += D[(long long)lo * k + hi] * rx[j];
-                }
-                rb[i] = a;
-            }
-        } else {
-            for (int r = threadIdx.x; r < k; r += BT) rb[r] = rx[r];
-        }
-        __syncthreads();
-        for (int j = threadIdx.x; j < n; j += BT) {
-            T s0 = 0, s1 = 0, s2 = 0, s3 = 0;  // four loads in flight, fixed order
-            int r = 0;
-            for (; r + 3 < k; r += 4) {
-                s0 += R[(long long)r * n + j] * (T)rb[r];
-                s1 += R[(long long)(r + 1) * n + j] * (T)rb[r + 1];
-                s2 += R[(long long)(r + 2) * n + j] * (T)rb[r + 2];
-                s3 += R[(long long)(r + 3) * n + j] * (T)rb[r + 3];
-            }
-            for (; r < k; ++r) s0 += R[(long long)r * n + j] * (T)rb[r];
-            qx[j] = qd[j] * x[j] + ((s0 + s1) + (s2 + s3));
+        low_rank_u(x);
+        for (int p = threadIdx.x; p < I.pn / 2; p += BT) {
+            T v[2];
+            low_rank_columns(p, v);
+            const auto q2 = load_pair(qd + 2 * p), x2 = load_pair(x + 2 * p);
+            store_pair(qx + 2 * p, q2[0] * x2[0] + v[0], q2[1] * x2[1] + v[1]);
         }
         __syncthreads();
     }
@@ -356,72 +628,102 @@ struct State {
     double max_pray, max_dray, pray_lin_obj, dray_obj;
 };
 
-// Projected BB inner solve of the primal prox (reference src/pdhg_core_op.cu:495-669).
+// Projected BB inner solve of the primal prox (reference
+// src/pdhg_core_op.cu:495-669).  A thread owns the column pairs tid, tid + BT,
+// ... of every vector throughout, so that a body is two passes: the gradient
+// step with R'u and the curvature, and the step itself with its norm (and the
+// new x_p staged).  Padding columns are zero in R and in every vector, with
+// bounds 0, and stay zero.
 template <class T, int BT> __device__ __noinline__ void bb_prox(const Ctx<T, BT> &C, State &S, double tau) {
     const Params &P = *C.P;
-    const int n = C.I.n;
-    T *x = C.nv(vX), *xp = C.nv(vXP), *xr = C.nv(vXR), *grad = C.nv(vGR), *dirn = C.nv(vDIR), *qx = C.nv(vQX),
-           *pb = C.nv(vPB), *md = C.nv(vMD), *mi = C.nv(vMI);
-    const T *c = C.nv(vC), *lb = C.nv(vLB), *ub = C.nv(vUB), *aty = C.nv(vATY), *dh = C.nv(vDH);
+    const int n = C.I.n, half = C.I.pn / 2;
+    T *x = C.nv(vX), *xp = C.nv(vXP), *xr = C.nv(vXR), *grad = C.nv(vGR), *dirn = C.nv(vDIR), *md = C.nv(vMD),
+      *mi = C.nv(vMI);
+    const T *c = C.nv(vC), *lb = C.nv(vLB), *ub = C.nv(vUB), *aty = C.nv(vATY), *dh = C.nv(vDH), *qd = C.nv(vQD);
     const double inv = 1.0 / tau;
     double a0 = 1.0 / inv;
     const bool pre = P.precond != 0;
     if (pre && S.cached_inv_tau != inv) {
         double sacc = 0.0;
-        for (int i = threadIdx.x; i < n; i += BT) {
-            double mm = dh[i] + inv;
-            if (mm <= 0.0) mm = 1.0;
-            md[i] = mm;
-            mi[i] = 1.0 / mm;
-            sacc += fabs(mm);
-        }
+        for (int p = threadIdx.x; p < half; p += BT)
+            for (int i = 2 * p; i < 2 * p + 2 && i < n; ++i) {
+                double mm = dh[i] + inv;
+                if (mm <= 0.0) mm = 1.0;
+                md[i] = mm;
+                mi[i] = 1.0 / mm;
+                sacc += fabs(mm);
+            }
         const double sum = C.red.sum(sacc);
         S.cached_inv_tau = inv;
         S.tol_scale = n > 0 ? sqrt(sum / (double)n) : 1.0;
     }
     if (pre) a0 *= S.tol_scale * S.tol_scale;
-    C.obj_product(x, qx);
-    for (int i = threadIdx.x; i < n; i += BT) {
-        const double g = qx[i] + c[i] - aty[i];
-        double nx = pre ? x[i] - a0 * mi[i] * g : x[i] - a0 * g;
-        nx = clampd(nx, lb[i], ub[i]);
-        xp[i] = nx;
-        grad[i] = g;
-        dirn[i] = nx - x[i];
-    }
+    // The step from `from` (x or x_p) along -scale [M^-1] g for pair p; returns its term of |s|^2 or s'Ms.
+    auto step = [&](int p, const T *from, double scale, double g0, double g1) {
+        const auto f2 = load_pair(from + 2 * p), l2 = load_pair(lb + 2 * p), u2 = load_pair(ub + 2 * p);
+        double w0 = 1.0, w1 = 1.0, m0 = 1.0, m1 = 1.0;
+        if (pre) {
+            const auto i2 = load_pair(mi + 2 * p), d2 = load_pair(md + 2 * p);
+            w0 = i2[0];
+            w1 = i2[1];
+            m0 = d2[0];
+            m1 = d2[1];
+        }
+        const T n0 = (T)clampd(f2[0] - scale * w0 * g0, l2[0], u2[0]);
+        const T n1 = (T)clampd(f2[1] - scale * w1 * g1, l2[1], u2[1]);
+        const T d0 = n0 - f2[0], d1 = n1 - f2[1];
+        store_pair(xp + 2 * p, n0, n1);
+        store_pair(dirn + 2 * p, d0, d1);
+        if (C.stage_room) store_pair_lds<T>(2 * p, n0, n1);
+        const double s0 = (double)d0 * (m0 * (double)d0), s1 = (double)d1 * (m1 * (double)d1);
+        return s0 + (2 * p + 1 < n ? s1 : 0.0);
+    };
+    C.stage(x);
     __syncthreads();
+    C.low_rank_u(x);
+    double nacc = 0.0;
+    for (int p = threadIdx.x; p < half; p += BT) {
+        const auto c2 = load_pair(c + 2 * p), a2 = load_pair(aty + 2 * p), q2 = load_pair(qd + 2 * p),
+                   x2 = load_pair(x + 2 * p);
+        T v[2];
+        C.low_rank_columns(p, v);
+        const T qx0 = q2[0] * x2[0] + v[0], qx1 = q2[1] * x2[1] + v[1];
+        const double g0 = (double)qx0 + (double)c2[0] - (double)a2[0], g1 = (double)qx1 + (double)c2[1] - (double)a2[1];
+        store_pair(grad + 2 * p, (T)g0, (T)g1);
+        nacc += step(p, x, a0, g0, g1);
+    }
     int it = 1;
     while (it < P.inner_limit) {
-        double stms = 0.0, nrm;
-        if (pre) {
-            stms = C.red.dot(n, [&](int i) { return dirn[i] * (md[i] * dirn[i]); });
-            nrm = sqrt(stms);
-        } else {
-            nrm = sqrt(C.red.dot(n, [&](int i) { return dirn[i] * dirn[i]; }));
-        }
+        const double s2 = C.red.sum(nacc), nrm = sqrt(s2);
         if (nrm <= S.inner_tol) break;
-        C.obj_product(xp, qx);
+        C.low_rank_u(xp);
         double tacc = 0.0;
-        for (int i = threadIdx.x; i < n; i += BT) {
-            const double last = grad[i];
-            const double cur = qx[i] + c[i] - aty[i] + inv * (xp[i] - x[i]);
-            pb[i] = cur - last;
-            grad[i] = cur;
-            tacc += dirn[i] * pb[i];
+        for (int p = threadIdx.x; p < half; p += BT) {
+            const auto c2 = load_pair(c + 2 * p), a2 = load_pair(aty + 2 * p), q2 = load_pair(qd + 2 * p),
+                       x2 = load_pair(x + 2 * p), p2 = load_pair(xp + 2 * p), g2 = load_pair(grad + 2 * p),
+                       d2 = load_pair(dirn + 2 * p);
+            T v[2];
+            C.low_rank_columns(p, v);
+            const T qx0 = q2[0] * p2[0] + v[0], qx1 = q2[1] * p2[1] + v[1];
+            const double cur0 = (double)qx0 + (double)c2[0] - (double)a2[0] + inv * ((double)p2[0] - (double)x2[0]);
+            const double cur1 = (double)qx1 + (double)c2[1] - (double)a2[1] + inv * ((double)p2[1] - (double)x2[1]);
+            store_pair(grad + 2 * p, (T)cur0, (T)cur1);
+            tacc += (double)d2[0] * (double)(T)(cur0 - (double)g2[0]);
+            if (2 * p + 1 < n) tacc += (double)d2[1] * (double)(T)(cur1 - (double)g2[1]);
         }
         const double tmp = C.red.sum(tacc);
-        const double alpha = pre ? stms / tmp : (nrm * nrm) / tmp;
-        for (int i = threadIdx.x; i < n; i += BT) {
-            const double cur = xp[i];
-            double nx = pre ? cur - alpha * mi[i] * grad[i] : cur - alpha * grad[i];
-            nx = clampd(nx, lb[i], ub[i]);
-            dirn[i] = nx - cur;
-            xp[i] = nx;
+        const double alpha = pre ? s2 / tmp : (nrm * nrm) / tmp;
+        nacc = 0.0;
+        for (int p = threadIdx.x; p < half; p += BT) {
+            const auto g2 = load_pair(grad + 2 * p);
+            nacc += step(p, xp, alpha, (double)g2[0], (double)g2[1]);
         }
-        __syncthreads();
         it++;
     }
-    for (int i = threadIdx.x; i < n; i += BT) xr[i] = 2.0 * xp[i] - x[i];
+    for (int p = threadIdx.x; p < half; p += BT) {
+        const auto p2 = load_pair(xp + 2 * p), x2 = load_pair(x + 2 * p);
+        store_pair(xr + 2 * p, (T)(2.0 * (double)p2[0] - (double)x2[0]), (T)(2.0 * (double)p2[1] - (double)x2[1]));
+    }
     __syncthreads();
     S.inner_total += it - 1;
     if (!std::is_same<T, double>::value) S.sat = (P.inner_limit > 1 && it >= P.inner_limit) ? S.sat + 1 : 0;
@@ -752,7 +1054,7 @@ template <class T, int BT>
 __global__ void __launch_bounds__(BT) batch_solve_kernel(const Params *P, const Inst *insts, const int *ipool,
                                                           const T *vpool, const double *dpool, T *slabs,
                                                           double *wslabs, const Cone *cones, State *states, Out *out,
-                                                          int budget) {
+                                                          int budget, int lds_bytes) {
     __shared__ double lds[2 * kBW];
     State S = states[blockIdx.x];
     if (S.reason != TERMINATION_REASON_UNSPECIFIED) return;
@@ -764,6 +1066,8 @@ __global__ void __launch_bounds__(BT) batch_solve_kernel(const Params *P, const 
     C.aci = ipool + C.I.a_ci;
     C.atrp = ipool + C.I.at_rp;
     C.atci = ipool + C.I.at_ci;
+    C.ach = ipool + C.I.a_chunk;
+    C.atch = ipool + C.I.at_chunk;
     C.av = vpool + C.I.a_v;
     C.atv = vpool + C.I.at_v;
     C.R = vpool + C.I.rdense;
@@ -772,6 +1076,18 @@ __global__ void __launch_bounds__(BT) batch_solve_kernel(const Params *P, const 
     C.W = wslabs + C.I.wvec;
     C.cones = cones + C.I.cone0;
     C.red.lds = lds;
+    // products stage their vector when it takes at most half of what a chunk
+    // leaves; as many rows of R stay as fit behind both
+    const int left = (lds_bytes - 2 * kMaxRank * (int)sizeof(double)) / (int)sizeof(T) - kChunk;
+    const int widest = max(C.I.pn, C.I.pm);
+    C.stage_room = widest <= left / 2 ? widest : 0;
+    C.room = C.stage_room + kChunk;
+    C.resident = C.I.qkind == kQLowRank ? min(C.I.k, (left - C.stage_room) / max(C.I.pn, 1)) : 0;
+    for (int e = 2 * (int)threadIdx.x; e < C.resident * C.I.pn; e += 2 * BT) {
+        const auto v = load_pair(C.R + e);
+        store_pair_lds<T>(C.room + e, v[0], v[1]);
+    }
+    __syncthreads();
     const int ef = P->ef;
     for (int pass = 0; pass < budget; ++pass) {
         if (!(S.total < P->iteration_limit)) {
