@@ -15,6 +15,7 @@
 // All cone arithmetic is FP64, whatever the storage type X of the vectors.
 #pragma once
 
+#include <algorithm>
 #include <cfloat>
 
 #include "dev_common.hpp"
@@ -954,9 +955,9 @@ constexpr int kPsdMaxSweeps = 60;
 // any (phase 2); the larger workgroup hides more latency per round and fits
 // 128 VGPRs with the smaller chunks.
 constexpr int kPsdThreads = 512, kPsdThreadsLarge = 1024;
-// V' columns per wave when V' is held in registers during the sweeps (the
-// 1024-thread form up to order 128)
-constexpr int kPsdRegCols = 8, kPsdRegMinOrder = 96;
+// Orders up to this are swept by position (psd_positions_kernel), with V' in
+// registers: kPsdRegCols columns per wave.
+constexpr int kPsdPosOrder = 128, kPsdRegCols = 8;
 template <int NT> struct PsdChunks {
     static constexpr int a = NT >= 1024 ? 2 : 4, v = NT >= 1024 ? 4 : 8;
 };
@@ -1149,27 +1150,6 @@ __global__ void __launch_bounds__(NT) psd_project_kernel(X *v, const PsdBlock *b
     // cover more pairs than threads
     const int tpp = nt >= np ? nt / np : 1, pstride = nt / tpp;
     const int nrp = (np + 1) / 2, tpr = nt >= nrp ? nt / nrp : 1, rstride = nt / tpr;
-    // V' in registers (the 1024-thread form at orders 97 to 128): lane L of
-    // every wave holds rows lu, ld of V' (the pair at position L of the
-    // round robin) for its wave's kPsdRegCols columns.  After each round
-    // the rows move one position along the circle (the up rows one lane
-    // right, the down rows one lane left, position 0's up row fixed), the
-    // same pairing as the circle ordering, so V' needs no memory round trip
-    // in a round.  Elsewhere V' stays in Vt and pairs come from the formula
-    // (below order 97 the LDS update is the cheaper: the shifts cost the
-    // same whatever the order).
-    const bool vreg = NT >= kPsdThreadsLarge && np <= kWave && kp > kPsdRegMinOrder &&
-                      kp <= (NT / kWave) * kPsdRegCols;
-    const int lane = tid % kWave, wcol = (tid / kWave) * kPsdRegCols;
-    int lu = 2 * lane, ld = 2 * lane + 1;
-    double vu[kPsdRegCols], vd[kPsdRegCols];
-#pragma unroll
-    for (int j = 0; j < kPsdRegCols; ++j) {
-        const int c = wcol + j;
-        const bool ok = vreg && lane < np && c < kp;
-        vu[j] = ok ? Vt[(size_t)lu * kp + c] : 0.0;
-        vd[j] = ok ? Vt[(size_t)ld * kp + c] : 0.0;
-    }
     bool converged = false;
     for (int sweep = 0; sweep <= kPsdMaxSweeps; ++sweep) {
         double off = 0.0, tot = 0.0;
@@ -1204,17 +1184,7 @@ __global__ void __launch_bounds__(NT) psd_project_kernel(X *v, const PsdBlock *b
         for (int t = 0; t < m; ++t) {
             // phase 1: the round's pairs and rotations
             for (int i = tid; i < np; i += nt) {
-                int a, b;
-                if (vreg) {
-                    a = lu;  // i == lane: wave 0 holds position i
-                    b = ld;
-                } else if (i == 0) {
-                    a = t;
-                    b = m;
-                } else {
-                    a = (t + i) % m;
-                    b = (t - i + m) % m;
-                }
+                const int a = i == 0 ? t : (t + i) % m, b = i == 0 ? m : (t - i + m) % m;
                 const int p = a < b ? a : b, q = a < b ? b : a;
                 const double apq = A[q * (q + 1) / 2 + p];
                 double c = 1.0, s = 0.0;
@@ -1230,8 +1200,7 @@ __global__ void __launch_bounds__(NT) psd_project_kernel(X *v, const PsdBlock *b
                 pq[2 * i + 1] = q;
             }
             __syncthreads();
-            // phase 2: the 2x2 blocks, then the rows of V' (in Vt or in
-            // registers).
+            // phase 2: the 2x2 blocks, then the rows of V'.
             // The 2x2 blocks: a block row pair holds block rows
             // rp and np - 1 - rp (np + 1 blocks; the middle row alone when np
             // is odd); its tpr threads take every tpr-th block, loading
@@ -1280,7 +1249,7 @@ __global__ void __launch_bounds__(NT) psd_project_kernel(X *v, const PsdBlock *b
             }
             // rows p, q of V' in Vt: the tpp threads of a pair take every
             // tpp-th column, kPsdChunkV columns loaded before any is stored
-            for (int P = vreg ? np : tid / tpp; P < np; P += pstride) {
+            for (int P = tid / tpp; P < np; P += pstride) {
                 const double c = cs[2 * P], s = cs[2 * P + 1];
                 if (s == 0.0) continue;
                 double *vp = Vt + (size_t)pq[2 * P] * kp, *vq = Vt + (size_t)pq[2 * P + 1] * kp;
@@ -1301,52 +1270,8 @@ __global__ void __launch_bounds__(NT) psd_project_kernel(X *v, const PsdBlock *b
                     }
                 }
             }
-            if (vreg) {
-                // this round's rotation of the lane's two rows (p = min(lu, ld))
-                const double c = lane < np ? cs[2 * lane] : 1.0, s = lane < np ? cs[2 * lane + 1] : 0.0;
-                if (s != 0.0) {
-                    const bool up_is_p = lu < ld;
-#pragma unroll
-                    for (int j = 0; j < kPsdRegCols; ++j) {
-                        const double a = up_is_p ? vu[j] : vd[j], b = up_is_p ? vd[j] : vu[j];
-                        const double na = c * a - s * b, nb2 = s * a + c * b;
-                        vu[j] = up_is_p ? na : nb2;
-                        vd[j] = up_is_p ? nb2 : na;
-                    }
-                }
-                // next round's positions (a single pair stays in place);
-                // columns past kp are skipped by whole waves
-                const int from_prev = lane > 0 ? lane - 1 : 0, from_next = lane + 1 < kWave ? lane + 1 : lane;
-#pragma unroll
-                for (int j = 0; j < kPsdRegCols; ++j) {
-                    if (wcol + j >= kp) break;
-                    const double up_prev = __shfl(vu[j], from_prev, kWave);
-                    const double dn_next = __shfl(vd[j], from_next, kWave);
-                    const double dn0 = __shfl(vd[j], 0, kWave);
-                    const double nu = lane == 0 ? vu[j] : (lane == 1 ? dn0 : up_prev);
-                    vd[j] = lane == np - 1 ? (np > 1 ? vu[j] : vd[j]) : dn_next;
-                    vu[j] = nu;
-                }
-                const int lu_prev = __shfl(lu, from_prev, kWave), ld_next = __shfl(ld, from_next, kWave);
-                const int ld0 = __shfl(ld, 0, kWave);
-                const int nlu = lane == 0 ? lu : (lane == 1 ? ld0 : lu_prev);
-                ld = lane == np - 1 ? (np > 1 ? lu : ld) : ld_next;
-                lu = nlu;
-            }
             __syncthreads();
         }
-    }
-    if (vreg) {
-        // V' back to Vt, rows at the lanes' final positions
-#pragma unroll
-        for (int j = 0; j < kPsdRegCols; ++j) {
-            const int c = wcol + j;
-            if (lane < np && c < kp) {
-                Vt[(size_t)lu * kp + c] = vu[j];
-                Vt[(size_t)ld * kp + c] = vd[j];
-            }
-        }
-        __syncthreads();
     }
     // keep V' for the next call (identity after a failure)
     if (vlds || !converged)
@@ -1385,6 +1310,310 @@ __global__ void __launch_bounds__(NT) psd_project_kernel(X *v, const PsdBlock *b
                 v[start + c * k - c * (c - 1) / 2 + (r - c)] = (X)val;
             }
     }
+}
+
+// ---------------- PSD cone up to order kPsdPosOrder: sweeps by position ----------------
+//
+// The same projection (warm transform, round-robin Jacobi, positive part) with
+// the matrix stored by the pairs' positions in the tournament instead of by
+// index: position L holds an up and a down element, block (P, Q), P >= Q, of
+// positions the four entries uu, ud, du, dd (a diagonal block uu, ud, dd), each
+// kind in a plane of its own with consecutive Q adjacent.  A round rotates
+// every block and writes its entries to where the elements stand in the next
+// round (position 0's up fixed, the up row one to the right, the down row one
+// to the left), into the other of two buffers.  A thread's blocks and the
+// places it writes to are the same in every round, so that a round has no
+// index arithmetic, and a wave's reads and nearly all of its writes are
+// consecutive.  After a sweep every element is back at its place.  A round is
+// bound by LDS traffic (order 128: 133 KB) and the vector unit (the moves of
+// V'), below order 64 by the rotation's chain and the two barriers.  Measured
+// (one block, a sequence of nearby points, us per point, psd_project_kernel
+// with scattered 2x2 blocks / here): order 16 135 / 73, 32 315 / 154,
+// 64 827 / 380, 96 2162 / 719, 128 3323 / 1280.  (Updating V' during the next
+// round's rotations instead of beside the blocks: 128 1386.)
+//
+// V' stays in registers: the last np lanes of each wave hold the rows of the
+// np positions' elements for the wave's kPsdRegCols columns and pass them on
+// with DPP wave shifts.  Dynamic LDS: the two buffers (133 KB at order 128); V' for the
+// products before and after the sweeps takes the same place.
+inline size_t psd_positions_lds(int k) {
+    const size_t kp = (size_t)(k + (k & 1)), np = kp / 2, nb = np * (np + 1) / 2;
+    return (std::max(8 * nb, kp * kp) + 2 * np + kp) * sizeof(double);
+}
+
+constexpr int kDppWaveShr1 = 0x138, kDppWaveShl1 = 0x130;  // lane i takes lane i - 1's / i + 1's value
+
+// The same moves, lanes without a source taking `old`.
+template <int Ctrl> __device__ __forceinline__ double psd_shift(double old, double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned long long o = (unsigned long long)__double_as_longlong(old);
+    const int lo = __builtin_amdgcn_update_dpp((int)(unsigned)o, (int)(unsigned)b, Ctrl, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(unsigned)(o >> 32), (int)(unsigned)(b >> 32), Ctrl, 0xf, 0xf, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// 1 / sqrt(x), x in [0.25, 8]: the hardware's estimate, two Newton steps.
+__device__ __forceinline__ double psd_rsqrt(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    for (int i = 0; i < 2; ++i) {
+        const double e = fma(-x * y, y, 1.0);
+        y = fma(0.5 * y, e, y);
+    }
+    return y;
+}
+
+// Jacobi rotation (c, s) that takes the off-diagonal a of [[u, a], [a, d]] to
+// zero, |angle| <= pi / 4: with h = (d - u) / 2 and r = sqrt(h^2 + a^2),
+// c^2 = (1 + |h| / r) / 2 and s = sign(h) a / (2 r c).  Two reciprocal roots
+// in a row instead of two quotients and two roots; h and a are brought to
+// [1/2, 1) by a power of two first, and c gets one correction toward
+// c^2 + s^2 = 1.
+__device__ __forceinline__ void psd_rotation(double u, double a, double d, double &c, double &s) {
+    c = 1.0;
+    s = 0.0;
+    if (a == 0.0) return;
+    double h = 0.5 * d - 0.5 * u;
+    const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(h), fabs(a)));
+    h = ldexp(h, e);
+    a = ldexp(a, e);
+    const double q = psd_rsqrt(fma(h, h, a * a));
+    const double cc = fma(0.5 * fabs(h), q, 0.5), ic = psd_rsqrt(cc);
+    s = copysign(0.5, h) * a * q * ic;
+    c = cc * ic;
+    c = fma(0.5 * ic, fma(-s, s, fma(-c, c, 1.0)), c);
+}
+
+template <class X>
+__global__ void __launch_bounds__(kPsdThreadsLarge) psd_positions_kernel(X *v, const PsdBlock *blocks, double *work,
+                                                                          int site, const int *gate) {
+    if (gate && *gate == 0) return;
+    constexpr int kMaxW = kPsdThreadsLarge / kWave;
+    constexpr int kBlocksPerThread = (kPsdPosOrder / 2 * (kPsdPosOrder / 2 + 1) / 2 + kPsdThreadsLarge - 1) / kPsdThreadsLarge;
+    extern __shared__ double psd_lds[];
+    __shared__ double red[2 * kMaxW];
+    __shared__ int stop;
+    const PsdBlock blk = blocks[blockIdx.x];
+    const int start = blk.start, k = blk.order, tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    if (k == 1) {
+        if (tid == 0) v[start] = (X)fmax((double)v[start], 0.0);
+        return;
+    }
+    const int kp = k + (k & 1), np = kp / 2, nb = np * (np + 1) / 2, kk = kp * kp;
+    // whole waves that have neither columns of V' nor blocks leave (a barrier
+    // waits for the waves that are left)
+    const int W = min(kMaxW, max((kp + kPsdRegCols - 1) / kPsdRegCols, (nb + kWave - 1) / kWave)), NT = W * kWave;
+    if (wave >= W) return;
+    double *wb = work + blk.work, *Vkeep = wb + (size_t)site * kk, *F = wb + 2 * (size_t)kk, *S = wb + 3 * (size_t)kk;
+    double *Vl = psd_lds, *cur = psd_lds, *nxt = psd_lds + 4 * nb;
+    double *cs = psd_lds + max(8 * nb, kk), *lam = cs + 2 * np;
+
+    for (int i = tid; i < kk; i += NT) {
+        F[i] = 0.0;
+        Vl[i] = Vkeep[i];
+    }
+    __syncthreads();
+    for (int slot = tid; slot < k * (k + 1) / 2; slot += NT) {
+        int r, c;
+        psd_slot_rc(slot, k, r, c);
+        double val = (double)v[start + slot];
+        if (r != c) val *= kInvSqrt2;
+        F[r * kp + c] = val;
+        F[c * kp + r] = val;
+    }
+    __syncthreads();
+    // warm transform B = V' F V'^T: S = (V' F)^T, then the lower tiles of
+    // V' S; one 4 x 4 tile per thread covers the matrix
+    const int tiles = (kp + 3) / 4, ti = tid / tiles, tj = tid - ti * tiles;
+    double acc[4][4];
+    if (ti < tiles) {
+        psd_tile_xy(Vl, F, kp, 4 * ti, 4 * tj, acc);
+        for (int u = 0; u < 4; ++u)
+            for (int w = 0; w < 4; ++w)
+                if (4 * ti + u < kp && 4 * tj + w < kp) S[(4 * tj + w) * kp + 4 * ti + u] = acc[u][w];
+    }
+    __syncthreads();
+    const bool lower = ti < tiles && tj <= ti;
+    if (lower) psd_tile_xy(Vl, S, kp, 4 * ti, 4 * tj, acc);
+    const int wcol = wave * kPsdRegCols, pos = lane - (kWave - np);
+    double vu[kPsdRegCols], vd[kPsdRegCols];
+#pragma unroll
+    for (int j = 0; j < kPsdRegCols; ++j) {
+        const bool ok = pos >= 0 && wcol + j < kp;
+        vu[j] = ok ? Vl[2 * pos * kp + wcol + j] : 0.0;
+        vd[j] = ok ? Vl[(2 * pos + 1) * kp + wcol + j] : 0.0;
+    }
+    auto turn_v = [&]() {  // one round: the rotations, then the moves
+        if (wcol >= kp) return;
+        const double c = pos >= 0 ? cs[2 * pos] : 1.0, s = pos >= 0 ? cs[2 * pos + 1] : 0.0;
+#pragma unroll
+        for (int j = 0; j < kPsdRegCols; ++j) {
+            const double u = c * vu[j] - s * vd[j], d = s * vu[j] + c * vd[j];
+            const double up = psd_shift<kDppWaveShr1>(u, pos == 0 ? d : u);
+            vu[j] = pos == 0 ? u : up;
+            vd[j] = np == 1 ? d : psd_shift<kDppWaveShl1>(u, d);
+        }
+    };
+    __syncthreads();
+    if (lower)
+        for (int u = 0; u < 4; ++u)
+            for (int w = 0; w < 4; ++w) {
+                const int i = 4 * ti + u, j = 4 * tj + w;
+                if (i >= kp || j > i) continue;
+                const int P = i / 2, Q = j / 2, plane = P == Q && i != j ? 1 : 2 * (i & 1) + (j & 1);
+                cur[plane * nb + P * (P + 1) / 2 + Q] = acc[u][w];
+            }
+    // this thread's blocks: positions (P, Q), and where the four entries go
+    int bp[kBlocksPerThread], bq[kBlocksPerThread], dst[kBlocksPerThread][4];
+    auto place = [&](int x, int L, int &x2, int &L2) {  // next round's row (0 up, 1 down) and position
+        x2 = x;
+        L2 = L;
+        if (np == 1 || (x == 0 && L == 0)) return;
+        if (x == 0) {
+            if (L == np - 1) x2 = 1;
+            else L2 = L + 1;
+        } else if (L == 0) {
+            x2 = 0;
+            L2 = 1;
+        } else L2 = L - 1;
+    };
+#pragma unroll
+    for (int j = 0; j < kBlocksPerThread; ++j) {
+        const int b = tid + j * NT;
+        bp[j] = b < nb ? psd_tri_row(b) : -1;
+        bq[j] = b < nb ? b - bp[j] * (bp[j] + 1) / 2 : 0;
+        for (int e = 0; e < 4; ++e) {
+            int x, y, P, Q;
+            place(e >> 1, max(bp[j], 0), x, P);
+            place(e & 1, bq[j], y, Q);
+            const int plane = P == Q && x != y ? 1 : P >= Q ? 2 * x + y : 2 * y + x;
+            const int hi = max(P, Q), lo = min(P, Q);
+            dst[j][e] = plane * nb + hi * (hi + 1) / 2 + lo;
+        }
+    }
+    __syncthreads();
+
+    bool converged = false;
+    for (int sweep = 0; sweep <= kPsdMaxSweeps; ++sweep) {
+        double off = 0.0, tot = 0.0;
+#pragma unroll
+        for (int j = 0; j < kBlocksPerThread; ++j) {
+            if (bp[j] < 0) continue;
+            const double *b = cur + tid + j * NT;
+            const double uu = b[0], ud = b[nb], dd = b[3 * nb];
+            if (bp[j] == bq[j]) {
+                tot += uu * uu + dd * dd;
+                off += 2.0 * (ud * ud);
+            } else {
+                const double du = b[2 * nb];
+                off += 2.0 * ((uu * uu + ud * ud) + (du * du + dd * dd));
+            }
+        }
+        off = wave_total(off);
+        tot = wave_total(tot);
+        if (lane == 0) {
+            red[2 * wave] = off;
+            red[2 * wave + 1] = tot;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            double o = 0.0, s = 0.0;
+            for (int w = 0; w < W; ++w) {
+                o += red[2 * w];
+                s += red[2 * w + 1];
+            }
+            s += o;
+            stop = (o <= 1e-30 * s || o == 0.0) ? 1 : 0;
+        }
+        __syncthreads();
+        if (stop) {
+            converged = true;
+            break;
+        }
+        if (sweep == kPsdMaxSweeps) break;
+        for (int t = 0; t < kp - 1; ++t) {
+            if (tid < np) {  // the rotation of each position's two elements
+                const double *b = cur + tid * (tid + 1) / 2 + tid;
+                const double a = b[nb];
+                double c, s;
+                psd_rotation(b[0], a, b[3 * nb], c, s);
+                cs[2 * tid] = c;
+                cs[2 * tid + 1] = s;
+            }
+            __syncthreads();
+            double e[kBlocksPerThread][4];
+#pragma unroll
+            for (int j = 0; j < kBlocksPerThread; ++j)
+                if (bp[j] >= 0)
+                    for (int q = 0; q < 4; ++q) e[j][q] = cur[q * nb + tid + j * NT];
+#pragma unroll
+            for (int j = 0; j < kBlocksPerThread; ++j) {
+                if (bp[j] < 0) continue;
+                const double c1 = cs[2 * bp[j]], s1 = cs[2 * bp[j] + 1], c2 = cs[2 * bq[j]], s2 = cs[2 * bq[j] + 1];
+                if (bp[j] == bq[j]) {
+                    const double uu = e[j][0], ud = e[j][1], dd = e[j][3];
+                    const double mu = c1 * uu - s1 * ud, mud = c1 * ud - s1 * dd;
+                    const double md = s1 * uu + c1 * ud, mdd = s1 * ud + c1 * dd;
+                    nxt[dst[j][0]] = c1 * mu - s1 * mud;
+                    nxt[dst[j][1]] = 0.0;
+                    nxt[dst[j][3]] = s1 * md + c1 * mdd;
+                    continue;
+                }
+                const double m00 = c1 * e[j][0] - s1 * e[j][2], m01 = c1 * e[j][1] - s1 * e[j][3];
+                const double m10 = s1 * e[j][0] + c1 * e[j][2], m11 = s1 * e[j][1] + c1 * e[j][3];
+                nxt[dst[j][0]] = c2 * m00 - s2 * m01;
+                nxt[dst[j][1]] = s2 * m00 + c2 * m01;
+                nxt[dst[j][2]] = c2 * m10 - s2 * m11;
+                nxt[dst[j][3]] = s2 * m10 + c2 * m11;
+            }
+            turn_v();
+            __syncthreads();
+            double *swap = cur;
+            cur = nxt;
+            nxt = swap;
+        }
+    }
+    for (int e = tid; e < kp; e += NT) {
+        const int L = e / 2;
+        lam[e] = fmax(cur[(e & 1 ? 3 * nb : 0) + L * (L + 1) / 2 + L], 0.0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPsdRegCols; ++j)
+        if (pos >= 0 && wcol + j < kp) {
+            Vl[2 * pos * kp + wcol + j] = vu[j];
+            Vl[(2 * pos + 1) * kp + wcol + j] = vd[j];
+        }
+    __syncthreads();
+    // keep V' for the next call (identity after a failure)
+    for (int i = tid; i < kk; i += NT) Vkeep[i] = converged ? Vl[i] : (i / kp == i % kp ? 1.0 : 0.0);
+    // svec of V'^T max(diag, 0) V' on the lower 4 x 4 tiles of k x k
+    const int nk = (k + 3) / 4, oi = tid / nk, oj = tid - oi * nk;
+    if (oi >= nk || oj > oi) return;
+    const int r0 = 4 * oi, c0 = 4 * oj;
+    for (int u = 0; u < 4; ++u)
+        for (int w = 0; w < 4; ++w) acc[u][w] = 0.0;
+    if (converged) {
+        for (int e = 0; e < kp; ++e) {
+            const double le = lam[e];
+            if (le == 0.0) continue;
+            const double *ve = Vl + e * kp;
+            double a[4], b[4];
+            for (int u = 0; u < 4; ++u) {
+                a[u] = r0 + u < k ? le * ve[r0 + u] : 0.0;
+                b[u] = c0 + u < k ? ve[c0 + u] : 0.0;
+            }
+            for (int u = 0; u < 4; ++u)
+                for (int w = 0; w < 4; ++w) acc[u][w] = fma(a[u], b[w], acc[u][w]);
+        }
+    }
+    for (int u = 0; u < 4; ++u)
+        for (int w = 0; w < 4; ++w) {
+            const int r = r0 + u, c = c0 + w;
+            if (r >= k || c > r) continue;
+            double val = converged ? acc[u][w] : NAN;
+            if (r != c) val *= kSqrt2;
+            v[start + c * k - c * (c - 1) / 2 + (r - c)] = (X)val;
+        }
 }
 
 // Elementwise helpers on cone slots, driven by a slot mask (kMaskCone on

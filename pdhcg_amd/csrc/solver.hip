@@ -131,7 +131,9 @@ struct RunStats {
 // orders first.
 struct PsdSet {
     int count = 0;
+    int by_index = 0;           // the first ones run psd_project_kernel, the others psd_positions_kernel
     size_t lds = 0;             // dynamic LDS bytes per workgroup (the largest need)
+    size_t pos_lds = 0;         // the same for psd_positions_kernel
     PsdBlock *blocks = nullptr;
     double *work = nullptr;     // psd_work_doubles(order, mode) per block
 };
@@ -145,28 +147,35 @@ inline size_t psd_lds_budget() {
     return lds > 1024 ? (size_t)lds - 1024 : 0;
 }
 
-// Launches the PSD projection of every block; `site` selects which kept
-// eigenvector set warm-starts it (0: the iterate, 1: the dual residual).
-// Dynamic LDS above the default limit is requested once per instance.
-template <class X> void psd_launch(const PsdSet &g, X *v, int site, const int *gate, hipStream_t st) {
-    static bool raised[2] = {false, false};
-    if (!g.count) return;
-    // PDHCG_PSD_THREADS=512|1024 picks the workgroup size (default 1024)
+// PDHCG_PSD_THREADS=512|1024 picks the workgroup size of psd_project_kernel
+// (default 1024); 512 also sends every order to it.
+inline int psd_threads() {
     static const int threads = [] {
         const char *e = std::getenv("PDHCG_PSD_THREADS");
         return e && std::atoi(e) == 512 ? kPsdThreads : kPsdThreadsLarge;
     }();
-    auto go = [&](auto kernel, int which, int nt) {
-        if (!raised[which] && g.lds > 0) {
+    return threads;
+}
+
+// Launches the PSD projection of every block; `site` selects which kept
+// eigenvector set warm-starts it (0: the iterate, 1: the dual residual).
+// Dynamic LDS above the default limit is requested once per instance.
+template <class X> void psd_launch(const PsdSet &g, X *v, int site, const int *gate, hipStream_t st) {
+    static bool raised[3] = {false, false, false};
+    auto go = [&](auto kernel, int which, int nt, int first, int count, size_t lds) {
+        if (!count) return;
+        if (!raised[which] && lds > 0) {
             HIP_OK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)psd_lds_budget()));
             raised[which] = true;
         }
-        hipLaunchKernelGGL(kernel, dim3(g.count), dim3(nt), g.lds, st, v, (const PsdBlock *)g.blocks, g.work, site,
+        hipLaunchKernelGGL(kernel, dim3(count), dim3(nt), lds, st, v, (const PsdBlock *)g.blocks + first, g.work, site,
                            gate);
     };
-    if (threads == kPsdThreadsLarge) go(psd_project_kernel<X, kPsdThreadsLarge>, 1, kPsdThreadsLarge);
-    else go(psd_project_kernel<X, kPsdThreads>, 0, kPsdThreads);
+    if (psd_threads() == kPsdThreadsLarge)
+        go(psd_project_kernel<X, kPsdThreadsLarge>, 1, kPsdThreadsLarge, 0, g.by_index, g.lds);
+    else go(psd_project_kernel<X, kPsdThreads>, 0, kPsdThreads, 0, g.by_index, g.lds);
+    go(psd_positions_kernel<X>, 2, kPsdThreadsLarge, g.by_index, g.count - g.by_index, g.pos_lds);
 }
 
 class DevConeSet {
@@ -315,9 +324,9 @@ class DevConeSet {
                          [](const std::pair<int, int> &x, const std::pair<int, int> &y) { return x.first > y.first; });
         if (!ps.empty()) {
             const size_t budget = psd_lds_budget();
-            // PDHCG_PSD_MODE=1|2|3 moves V' (1), A (2) or both (3) to the work
-            // buffer on orders whose layout would fit LDS (the tests run every
-            // mode)
+            // PDHCG_PSD_MODE=1|2|3 sends every order to psd_project_kernel with V'
+            // (1), A (2) or both (3) in the work buffer also where its layout
+            // would fit LDS (the tests run every mode)
             const char *fm = std::getenv("PDHCG_PSD_MODE");
             std::vector<PsdBlock> hb(ps.size());
             long long work = 0;
@@ -334,7 +343,13 @@ class DevConeSet {
                 pb.pad = 0;
                 pb.work = work;
                 work += (long long)psd_work_doubles(pb.order, pb.mode);
-                pset.lds = std::max(pset.lds, psd_lds_bytes(pb.order, pb.mode));
+                if (!fm && pb.order <= kPsdPosOrder && psd_threads() == kPsdThreadsLarge &&
+                    psd_positions_lds(pb.order) <= budget) {
+                    pset.pos_lds = std::max(pset.pos_lds, psd_positions_lds(pb.order));
+                } else {
+                    pset.by_index = (int)i + 1;  // largest orders first
+                    pset.lds = std::max(pset.lds, psd_lds_bytes(pb.order, pb.mode));
+                }
             }
             pset.count = (int)hb.size();
             pset.blocks = up<PsdBlock>(hb, hb.size());
