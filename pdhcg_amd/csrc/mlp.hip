@@ -7,7 +7,8 @@
 //
 // Matrix product: C[M x N] = op(A)[M x K] op(B)[K x N], BF16 operands, op =
 // identity or transpose of a row-major array; M, N, K multiples of 16 (the
-// host pads).  A workgroup of four waves owns a 64 x 64 tile of C and walks K
+// host pads).  Products with few tiles go to gemm_small_kernel; the others to
+// gemm_kernel: a workgroup of four waves owns a 64 x 64 tile of C and walks K
 // in steps of 128 (few, large steps: the products here are small and each
 // step costs a memory round trip): each step's A and B tiles go global ->
 // registers (16-byte loads along the contiguous dimension) -> LDS
@@ -247,6 +248,186 @@ template <bool TA, bool TB, int EPI> __global__ void __launch_bounds__(256) gemm
     }
 }
 
+// The same products where gemm_kernel's 64 x 64 tiles are too few for the
+// chip: a workgroup of eight waves owns a 32 x 32 tile and takes K in chunks of
+// 1024, so that K = 1024 is one round trip to memory where gemm_kernel made
+// eight.  Wave w loads the chunk's steps of 32 numbered w, w + 8, ... (the next
+// chunk's while this one is multiplied) and puts them into LDS as the
+// instruction takes them, lane by lane; waves 0 to 3 then multiply one 16 x 16
+// block each, step after step, so that every sum is formed in gemm_kernel's
+// order and is bitwise the same, and all eight finish two results per thread.
+// An operand contiguous along k is loaded as it is used; of the others a lane
+// loads two neighbouring rows of op(A) (columns of op(B)) for its eight k and
+// sorts the halves with v_perm: block b of the two holds the indices 2 i + b.
+// Bound by the latency of its loads.  Measured (256 x 1024 results, us,
+// gemm_kernel / here): bias and GELU over K = 16 7.7 / 4.9, over 1024
+// 15.5 / 6.4; GELU's derivative over K = 1024 15.1 / 7.4, over 3008 26.7 / 15.9.
+constexpr int kSmallTile = 32, kSmallWaves = 8, kSmallLoads = 4, kSmallPitch = kSmallTile + 2;
+constexpr int kSmallSteps = kSmallWaves * kSmallLoads;  // steps of 32 k per chunk
+struct SmallLds {
+    uint4 ops[kSmallSteps][4][kWave];      // per step: op(A)'s two blocks, op(B)'s two
+    float tile[kSmallTile * kSmallPitch];  // the products, then the gradients
+    float csum[4][kSmallTile];
+    double loss[kSmallWaves];
+};
+struct SmallRaw {
+    unsigned v[8];
+};
+template <bool KMAJ> __device__ __forceinline__ void small_load(SmallRaw &r, const bf16 *P, int ld, int i0, int imax,
+                                                                int k0, int K) {
+    const int lane = threadIdx.x % kWave, l16 = lane % 16, k = k0 + 8 * (lane / 16);
+    if (KMAJ) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int i = i0 + 16 * b + l16;
+            uint4 x = {0u, 0u, 0u, 0u};
+            if (i < imax && k < K) x = *reinterpret_cast<const uint4 *>(P + (size_t)i * ld + k);
+            r.v[4 * b] = x.x;
+            r.v[4 * b + 1] = x.y;
+            r.v[4 * b + 2] = x.z;
+            r.v[4 * b + 3] = x.w;
+        }
+    } else {
+        const int i = i0 + 2 * l16;
+        const bool ok = i < imax && k < K;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            r.v[q] = ok ? *reinterpret_cast<const unsigned *>(P + (size_t)(k + q) * ld + i) : 0u;
+    }
+}
+template <bool KMAJ> __device__ __forceinline__ uint4 small_op(const SmallRaw &r, int b) {
+    unsigned x[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+        x[p] = KMAJ ? r.v[4 * b + p] : __builtin_amdgcn_perm(r.v[2 * p + 1], r.v[2 * p], b ? 0x07060302u : 0x05040100u);
+    return uint4{x[0], x[1], x[2], x[3]};
+}
+
+// Grid: (ceil(N / 32), ceil(M / 32)); 512 threads; dynamic LDS: SmallLds.
+template <bool TA, bool TB, int EPI> __global__ void __launch_bounds__(kSmallWaves *kWave) gemm_small_kernel(GemmArgs g) {
+    constexpr bool AK = !TA, BK = TB, kReduce = EPI == kBiasMse || EPI == kGeluBack;
+    extern __shared__ __align__(16) char small_lds[];
+    SmallLds &lds = *reinterpret_cast<SmallLds *>(small_lds);
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, l16 = lane % 16, kg = 4 * (lane / 16);
+    const int r0 = blockIdx.y * kSmallTile, c0 = blockIdx.x * kSmallTile;
+    SmallRaw a[kSmallLoads], b[kSmallLoads];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < kSmallLoads; ++u) {
+            const int k = k0 + 32 * (wave + kSmallWaves * u);
+            small_load<AK>(a[u], g.A, g.lda, r0, g.M, k, g.K);
+            small_load<BK>(b[u], g.B, g.ldb, c0, g.N, k, g.K);
+        }
+    };
+    load(0);
+    // the two neighbouring results this thread finishes, and what they need
+    const int rr = threadIdx.x / 16, cc = 2 * (threadIdx.x % 16), r = r0 + rr, c = c0 + cc;
+    const bool live = r < g.M && c < g.N;
+    const size_t o = (size_t)r * g.N + c;
+    float2 aux = {0.f, 0.f}, target = {0.f, 0.f};
+    if (live) {
+        if (EPI == kBiasGelu || EPI == kBias || EPI == kBiasMse) aux = *reinterpret_cast<const float2 *>(g.bias + c);
+        if (EPI == kGeluBack) aux = *reinterpret_cast<const float2 *>(g.Z + o);
+        if (EPI == kBiasMse) {
+            if (c < g.out) target.x = g.T[(size_t)r * g.out + c];
+            if (c + 1 < g.out) target.y = g.T[(size_t)r * g.out + c + 1];
+        }
+    }
+    const int bi = wave / 2, bj = wave % 2;  // the block of waves 0 to 3
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int kChunk = 32 * kSmallSteps;
+    for (int k0 = 0; k0 < g.K; k0 += kChunk) {
+        if (k0) __syncthreads();  // the last chunk has been multiplied
+#pragma unroll
+        for (int u = 0; u < kSmallLoads; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                lds.ops[wave + kSmallWaves * u][h][lane] = small_op<AK>(a[u], h);
+                lds.ops[wave + kSmallWaves * u][2 + h][lane] = small_op<BK>(b[u], h);
+            }
+        __syncthreads();
+        if (k0 + kChunk < g.K) load(k0 + kChunk);
+        if (wave < 4) {
+            auto step = [&](int i) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, lds.ops[i][bi][lane]),
+                                                              __builtin_bit_cast(b8, lds.ops[i][2 + bj][lane]), acc, 0,
+                                                              0, 0);
+            };
+            const int n = min(kSmallSteps, (g.K - k0 + 31) / 32);
+            if (n == kSmallSteps) {
+#pragma unroll
+                for (int i = 0; i < kSmallSteps; ++i) step(i);
+            } else {
+                for (int i = 0; i < n; ++i) step(i);
+            }
+        }
+    }
+    if (wave < 4)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int pr = AK ? 16 * bi + kg + q : 2 * (kg + q) + bi, pc = BK ? 16 * bj + l16 : 2 * l16 + bj;
+            lds.tile[pr * kSmallPitch + pc] = acc[q];
+        }
+    __syncthreads();
+    float2 &cell = *reinterpret_cast<float2 *>(&lds.tile[rr * kSmallPitch + cc]);
+    float2 v = cell;
+    float2 gr = {0.f, 0.f};  // kReduce: the two gradients
+    double lsum = 0.0;
+    if (live) {
+        float2 h = {0.f, 0.f};
+        if (EPI == kBiasGelu || EPI == kBias) {
+            v.x += aux.x;
+            v.y += aux.y;
+        }
+        if (EPI == kStore || EPI == kBiasGelu || EPI == kBias) *reinterpret_cast<float2 *>(g.C + o) = v;
+        if (EPI == kBiasGelu) h = {gelu(v.x), gelu(v.y)};
+        if (EPI == kBiasMse) {
+            const float dx = v.x + aux.x - target.x, dy = v.y + aux.y - target.y;
+            if (c < g.out) {
+                lsum += (double)dx * dx;
+                gr.x = g.scale * dx;
+            }
+            if (c + 1 < g.out) {
+                lsum += (double)dy * dy;
+                gr.y = g.scale * dy;
+            }
+        }
+        if (EPI == kGeluBack) gr = {v.x * gelu_grad(aux.x), v.y * gelu_grad(aux.y)};
+        if (kReduce) h = gr;
+        if (EPI != kStore && EPI != kBias)
+            *reinterpret_cast<unsigned *>(g.H + o) = (unsigned)to_bf16(h.x) | (unsigned)to_bf16(h.y) << 16;
+    }
+    if (kReduce) {
+        // column sums, in the order of gemm_kernel's lanes: rows 4 p .. 4 p + 3
+        // and 16 above them one after the other, then the four p in pairs
+        cell = gr;
+        if (EPI == kBiasMse) {
+            lsum = wave_sum(lsum);
+            if (lane == 0) lds.loss[wave] = lsum;
+        }
+        __syncthreads();
+        if (threadIdx.x < 4 * kSmallTile) {
+            const int p = threadIdx.x / kSmallTile, col = threadIdx.x % kSmallTile;
+            float t = 0.f;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) t += lds.tile[(16 * i + 4 * p + q) * kSmallPitch + col];
+            lds.csum[p][col] = t;
+        }
+        __syncthreads();
+        if (threadIdx.x < kSmallTile && c0 + (int)threadIdx.x < g.N)
+            g.colpart[(size_t)blockIdx.y * g.N + c0 + threadIdx.x] =
+                (lds.csum[0][threadIdx.x] + lds.csum[1][threadIdx.x]) +
+                (lds.csum[2][threadIdx.x] + lds.csum[3][threadIdx.x]);
+        if (EPI == kBiasMse && threadIdx.x == 0) {
+            double t = 0.0;
+            for (int w = 0; w < kSmallWaves; ++w) t += lds.loss[w];
+            g.lossp[blockIdx.y * gridDim.x + blockIdx.x] = t;
+        }
+    }
+}
+
 __global__ void to_bf16_kernel(const float *x, bf16 *y, long long n) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
         y[i] = to_bf16(x[i]);
@@ -278,7 +459,8 @@ struct FoldArgs {
     const float *colpart[3];
     float *gb[3];
     int cols[3];
-    int tiles;           // row tiles of the batch
+    int tiles[3];        // row tiles of the batch
+    bool half[3];        // tiles of 32 rows, not 64
     const double *lossp;
     int nloss;
     double scale;
@@ -290,7 +472,14 @@ __global__ void fold_kernel(FoldArgs f) {
         const int c = blockIdx.x * blockDim.x + threadIdx.x;
         if (c >= f.cols[s]) return;
         float acc = 0.0f;
-        for (int t = 0; t < f.tiles; ++t) acc += f.colpart[s][(size_t)t * f.cols[s] + c];
+        const float *p = f.colpart[s] + c;
+        const size_t cols = (size_t)f.cols[s];
+        // tiles of 32 rows in pairs first, as a tile of 64 adds its halves
+        if (f.half[s])
+            for (int t = 0; t < f.tiles[s]; t += 2)
+                acc += p[t * cols] + (t + 1 < f.tiles[s] ? p[(t + 1) * cols] : 0.0f);
+        else
+            for (int t = 0; t < f.tiles[s]; ++t) acc += p[t * cols];
         f.gb[s][c] = acc;
         return;
     }
@@ -355,9 +544,32 @@ struct Net {
 
 constexpr int kMaxSteps = 1 << 16;  // minibatches per epoch
 
+// Products of at most this many 64 x 64 tiles go to gemm_small_kernel: with
+// half the chip's units or more idle its shorter chain of round trips counts,
+// with more tiles gemm_kernel's, which reads each operand half as often.
+// Measured (us, gemm_kernel / gemm_small_kernel): 16 tiles over K = 256
+// 5.4 / 4.7, 64 tiles over K = 1024 15.1 / 7.4; 188 tiles over K = 1024
+// 18.1 / 22.8, 256 tiles over K = 256 6.0 / 12.7.
+constexpr long long kSmallUpTo = 128;
+
+inline int tiles_of(int n, int tile) { return (n + tile - 1) / tile; }
+
+// Tile edge of an M x N product.
+inline int tile_of(int M, int N) {
+    return (long long)tiles_of(M, kBM) * tiles_of(N, kBN) <= kSmallUpTo ? kSmallTile : kBM;
+}
+
 template <bool TA, bool TB, int EPI> void launch(hipStream_t st, const GemmArgs &a) {
-    dim3 grid((unsigned)((a.N + kBN - 1) / kBN), (unsigned)((a.M + kBM - 1) / kBM));
-    hipLaunchKernelGGL((gemm_kernel<TA, TB, EPI>), grid, dim3(256), 0, st, a);
+    const int tile = tile_of(a.M, a.N);
+    dim3 grid((unsigned)tiles_of(a.N, tile), (unsigned)tiles_of(a.M, tile));
+    if (tile == kSmallTile) {
+        static const hipError_t raised =
+            hipFuncSetAttribute((const void *)gemm_small_kernel<TA, TB, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)sizeof(SmallLds));
+        HIP_OK(raised);
+        hipLaunchKernelGGL((gemm_small_kernel<TA, TB, EPI>), grid, dim3(kSmallWaves * kWave), sizeof(SmallLds), st, a);
+    } else
+        hipLaunchKernelGGL((gemm_kernel<TA, TB, EPI>), grid, dim3(256), 0, st, a);
     HIP_OK(hipGetLastError());
 }
 
@@ -373,8 +585,6 @@ GemmArgs gemm_args(int M, int N, int K, const bf16 *A, int lda, const bf16 *B, i
     return a;
 }
 
-inline int row_tiles(int rows) { return (rows + kBM - 1) / kBM; }
-
 void free_batch(Net &n) {
     for (void *p : {(void *)n.xb, (void *)n.h1b, (void *)n.h2b, (void *)n.dyb, (void *)n.dz2b, (void *)n.dz1b,
                     (void *)n.z1, (void *)n.z2, (void *)n.y, (void *)n.t, (void *)n.colpart[0], (void *)n.colpart[1],
@@ -385,7 +595,7 @@ void free_batch(Net &n) {
 void ensure_batch(Net &n, int rows) {
     if (rows <= n.cap) return;
     free_batch(n);
-    const size_t r = (size_t)rows, H = (size_t)n.hidden, tiles = (size_t)row_tiles(rows);
+    const size_t r = (size_t)rows, H = (size_t)n.hidden, tiles = (size_t)tiles_of(rows, kSmallTile);
     n.xb = dnew<bf16>(r * n.in_p);
     n.z1 = dnew<float>(r * H);
     n.h1b = dnew<bf16>(r * H);
@@ -399,7 +609,7 @@ void ensure_batch(Net &n, int rows) {
     n.colpart[0] = dnew<float>(tiles * H);
     n.colpart[1] = dnew<float>(tiles * H);
     n.colpart[2] = dnew<float>(tiles * n.out_p);
-    n.lossp = dnew<double>(tiles * (size_t)((n.out_p + kBN - 1) / kBN));
+    n.lossp = dnew<double>(tiles * (size_t)tiles_of(n.out_p, kSmallTile));
     n.loss = dnew<double>(kMaxSteps);
     n.cap = rows;
 }
@@ -494,10 +704,12 @@ void backward(Net &n, int rows, double *loss) {
         f.colpart[l] = n.colpart[l];
         f.gb[l] = n.G + n.L[l].b;
         f.cols[l] = n.L[l].out;
+        const int tile = tile_of(rows, n.L[l].out);
+        f.tiles[l] = tiles_of(rows, tile);
+        f.half[l] = tile == kSmallTile;
     }
-    f.tiles = row_tiles(rows);
     f.lossp = n.lossp;
-    f.nloss = row_tiles(rows) * ((O + kBN - 1) / kBN);
+    f.nloss = f.tiles[2] * tiles_of(O, tile_of(rows, O));
     f.scale = 1.0 / ((double)rows * n.out);
     f.loss = loss;
     hipLaunchKernelGGL(fold_kernel, dim3((unsigned)((std::max(H, O) + 255) / 256), 4), dim3(256), 0, n.st, f);
