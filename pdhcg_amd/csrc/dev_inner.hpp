@@ -53,11 +53,14 @@ struct InnerExchange {
     long long wait;  // wall-clock ticks after which a wait gives up
 };
 
-// Arguments common to the forms.
+// Arguments common to the forms.  The Halpern update goes to x_next, not to x:
+// with an inner limit of 1 there is no exchange after the loads of x, and a
+// workgroup that starts late still reads other workgroups' columns of x.
 template <class X> struct InnerArgs {
     int n, limit, halpern;
     double alpha0, inv_tau, tol, w, rho;
-    X *x, *xp, *xr;
+    const X *x;
+    X *x_next, *xp, *xr;
     const X *x0, *c, *aty, *lb, *ub, *qdiag, *m_inv, *m_diag;
     InnerExchange ex;
     DevScalars *ds;
@@ -220,7 +223,7 @@ template <class X> struct InnerColumn {
         a.xr[i] = (X)ref;
         if (a.halpern) {
             const double refl = a.rho * ref + (1.0 - a.rho) * x;
-            a.x[i] = (X)(a.w * refl + (1.0 - a.w) * (double)a.x0[i]);
+            a.x_next[i] = (X)(a.w * refl + (1.0 - a.w) * (double)a.x0[i]);
         }
     }
 };

@@ -750,6 +750,7 @@ template <class V, class X> class Solver final : public SolverBase {
     InnerForm inner_form_ = kInnerLaunches;
     int inner_groups_ = 0, inner_cols_ = 0;
     size_t inner_lds_ = 0;
+    X *x_next_ = nullptr;  // where a resident inner solve leaves the Halpern update; then exchanged with x_
     InnerExchange exchange_ = {};
     // kInnerSparse: Q in row order, its rows cut into tasks
     int *qrow_task_ = nullptr, *qtask_start_ = nullptr, *qci_ = nullptr;
@@ -1255,6 +1256,7 @@ template <class V, class X> void Solver<V, X>::init_inner_form() {
         scalar = (size_t)2 * inner_groups_ * kInnerWaves;
     }
     if (inner_form_ == kInnerLaunches) return;
+    x_next_ = dalloc<X>(n_);
     exchange_.rows = dzeros<xword>(2 * rows);
     exchange_.total = dzeros<xword>(2 * total);
     exchange_.scalar = dzeros<xword>(2 * scalar);
@@ -1276,6 +1278,7 @@ template <class V, class X> void Solver<V, X>::inner_launch(double tau, bool fus
     a.w = w;
     a.rho = P_.reflection_coefficient;
     a.x = x_;
+    a.x_next = x_next_;
     a.xp = xp_;
     a.xr = xr_;
     a.x0 = x0_;
@@ -1327,8 +1330,8 @@ template <class V, class X> Solver<V, X>::~Solver() {
     pnAt_.release();
     void *ptrs[] = {qsdiag_, qdiag_, Rd_,     ddiag_,  ddense_,      u_,          rx_partials_, rx_counter_, rx_sums_,
                     rxv_,    lb_,    ub_,     c_,      cl_,          cu_,         g_,           cl_fin_,
-                    cu_fin_, lb_fin_, ub_fin_, con_rescale_, var_rescale_, x0_,     x_,           xp_,
-                    xr_,     y0_,    y_,      yp_,     yr_,          aty_,        ax_,          dslack_,
+                    cu_fin_, lb_fin_, ub_fin_, con_rescale_, var_rescale_, x0_,     x_,           x_next_,
+                    xp_,     xr_,     y0_,    y_,      yp_,     yr_,          aty_,        ax_,          dslack_,
                     dx_,     dy_,    qx_,     grad_,   dirn_,        mdiag_,      minv_,        diag_h_,
                     exchange_.rows, exchange_.total, exchange_.scalar, exchange_.seq, qrow_task_, qtask_start_, qci_, qv_,
                     red_partials_, ds_, snap_, pgp_, dres_, aff_d_, acomp_, aproj_, apres_, amem_};
@@ -1494,6 +1497,7 @@ template <class V, class X> void Solver<V, X>::bb_prox(double tau, bool fuse_hal
     }
     if (inner_form_ != kInnerLaunches) {
         inner_launch(tau, fuse_halpern, w);
+        if (fuse_halpern) std::swap(x_, x_next_);
         if (eval_) {  // the hand-over to FP64 counts inner solves that reached the limit
             HIP_OK(hipMemcpyAsync(bb_poll_, &ds_->bb_iter, sizeof(int), hipMemcpyDeviceToHost, st_));
             HIP_OK(hipStreamSynchronize(st_));
