@@ -23,9 +23,15 @@
 // such a kernel of kInnerPlainGroups (low rank: one workgroup per compute unit)
 // or kInnerSparseGroups (sparse: two per unit) workgroups, still fit the 256
 // compute units together.  Larger grids are launched cooperatively, which costs
-// about 18 us per launch more but guarantees residency.  A wait also ends
-// after kInnerWaitSeconds, marks the solve as failed (DevScalars::inner_fail,
-// reported by the host at its next read) and every workgroup leaves.
+// about 18 us per launch more but guarantees residency.
+//
+// A wait that lasts kInnerWaitSeconds gives up: it notes the launch's number in
+// DevScalars and clears inner_run, and every workgroup leaves.  All that changes
+// the state after an inner solve is gated by inner_run (later inner solves, the
+// dual step, the Halpern updates) and the inner solve itself writes no vector
+// that it reads, so the state stays that before the launch, and the host, at its
+// next read of the scalars, takes the loop back to there and goes on launch by
+// launch (Solver::rewind_inner).
 #pragma once
 
 #include "dev_kernels.hpp"
@@ -40,7 +46,9 @@ constexpr int kInnerPlainGroups = 8, kInnerSparseGroups = 16;
 constexpr int kInnerAllGroups = 16;            // low rank: every workgroup sums all partial rows up to here
 constexpr int kInnerMaxRank = 80;              // rows of R: ten per wave
 constexpr int kInnerSparseVars = 8192;         // x_p of the sparse form is held in LDS (64 KB)
-constexpr double kInnerWaitSeconds = 30.0;
+// Longer than other streams' kernels hold the chip as a rule; an exchange takes
+// microseconds.
+constexpr double kInnerWaitSeconds = 1.0;
 
 typedef unsigned long long xword;
 
@@ -58,6 +66,8 @@ struct InnerExchange {
 // workgroup that starts late still reads other workgroups' columns of x.
 template <class X> struct InnerArgs {
     int n, limit, halpern;
+    int launch;   // number of this inner solve
+    int give_up;  // 1: the last workgroup gives up at its first wait (tests)
     double alpha0, inv_tau, tol, w, rho;
     const X *x;
     X *x_next, *xp, *xr;
@@ -72,13 +82,26 @@ __device__ __forceinline__ void exchange_put(xword *slot, double v, unsigned seq
     __hip_atomic_store(slot + 1, t | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Where a wait that gave up is noted: for the host and the other workgroups
-// (device memory), and for this workgroup (LDS, read after its next barrier,
-// so that all its threads leave together).
+// What a wait that gives up does: notes it for the host and the other
+// workgroups (device memory), and for this workgroup (LDS, read after its next
+// barrier, so that all its threads leave together).
 struct InnerWait {
-    long long ticks;
-    int *fail, *group_fail;
+    long long ticks;  // negative: gives up at once
+    int launch;
+    DevScalars *ds;
+    int *group_fail;
+    __device__ bool others_gave_up() const {
+        return __hip_atomic_load(&ds->inner_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+    }
+    __device__ void give_up() const {
+        __hip_atomic_store(&ds->inner_gave_up, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ds->inner_run, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *group_fail = 1;
+    }
 };
+template <class X> __device__ __forceinline__ InnerWait inner_wait(const InnerArgs<X> &a, int *group_fail) {
+    return InnerWait{a.give_up && blockIdx.x + 1 == gridDim.x ? -1LL : a.ex.wait, a.launch, a.ds, group_fail};
+}
 
 // Waits for U values with sequence number `seq`, those at first, first + step,
 // ... below `count` (the others are 0), all loads in flight together (a load
@@ -99,16 +122,15 @@ __device__ __forceinline__ void exchange_get(const xword *slots, int first, int 
                 b[q] = __hip_atomic_load(slots + (size_t)i * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-        bool all = true;
+        bool all = w.ticks >= 0;
 #pragma unroll
         for (int q = 0; q < U; ++q) all = all && (unsigned)(a[q] >> 32) == seq && (unsigned)(b[q] >> 32) == seq;
         if (all) break;
-        if (polls % 256 == 0) {
+        if (polls % 256 == 0 || w.ticks < 0) {
             const long long now = wall_clock64();
             if (start == 0) start = now;
-            if (now - start > w.ticks || __hip_atomic_load(w.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                __hip_atomic_store(w.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                *w.group_fail = 1;
+            if (now - start > w.ticks || w.others_gave_up()) {
+                w.give_up();
 #pragma unroll
                 for (int q = 0; q < U; ++q) a[q] = b[q] = 0;
                 break;
@@ -118,6 +140,14 @@ __device__ __forceinline__ void exchange_get(const xword *slots, int first, int 
     }
 #pragma unroll
     for (int q = 0; q < U; ++q) v[q] = __longlong_as_double((long long)((b[q] << 32) | (a[q] & 0xffffffffull)));
+}
+
+// The flags before the first resident inner solve, and after one that gave up
+// (whose bodies the launches that take its place count again).
+__global__ void inner_reset_kernel(DevScalars *ds) {
+    if (ds->inner_gave_up && ds->inner_counted == ds->inner_gave_up) ds->inner_total -= ds->bb_iter - 1;
+    ds->inner_gave_up = 0;
+    ds->inner_run = 1;
 }
 
 // A sequence number kept between launches: read before the workgroup's first
@@ -252,7 +282,7 @@ __global__ void __launch_bounds__(kInnerThreads) inner_lowrank_kernel(InnerArgs<
                                                                        int dkind) {
     constexpr int NR = RW <= 1 ? 1 : RW <= 2 ? 2 : RW <= 4 ? 4 : RW <= 8 ? 8 : 16;
     __shared__ double xs[kInnerCols], part[kInnerWaves * kInnerCols];
-    __shared__ int group_fail;
+    __shared__ int group_fail, skip;
     __shared__ double dsum, us[kInnerMaxRank + 1], u2[kInnerMaxRank + 1], nw[kInnerWaves], dw[kInnerWaves];
     const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
     const int G = gridDim.x, g = blockIdx.x, rows = k + 1;
@@ -260,8 +290,11 @@ __global__ void __launch_bounds__(kInnerThreads) inner_lowrank_kernel(InnerArgs<
     const bool pre = a.m_inv != nullptr;
     unsigned seq_rows = inner_seq(a.ex.seq), seq_s = inner_seq(a.ex.seq + 1);
     DevScalars *ds = a.ds;
-    const InnerWait wait{a.ex.wait, &ds->inner_fail, &group_fail};
-    if (t == 0) group_fail = 0;
+    const InnerWait wait = inner_wait(a, &group_fail);
+    if (t == 0) {
+        group_fail = 0;
+        skip = G > 1 && wait.others_gave_up();
+    }
 
     V r[RW][kInnerColSets];
     const long long padded = (long long)rx_chunks(a.n) * kRxWaveCols;
@@ -372,7 +405,7 @@ __global__ void __launch_bounds__(kInnerThreads) inner_lowrank_kernel(InnerArgs<
     xs[t] = col.x;
     if (t < kInnerWaves) nw[t] = 0.0;
     __syncthreads();
-    if (!product()) return;
+    if (skip || !product()) return;
     double qx = transpose_product();
     if (a.qdiag) qx = qx + col.qd * col.x;
     double nv = col.first(qx, pre ? a.alpha0 * (ds->tol_scale * ds->tol_scale) : a.alpha0, pre);
@@ -411,6 +444,7 @@ __global__ void __launch_bounds__(kInnerThreads) inner_lowrank_kernel(InnerArgs<
     if (g == 0 && t == 0) {
         ds->bb_iter = it;
         ds->inner_total += it - 1;
+        ds->inner_counted = a.launch;
         a.ex.seq[0] = seq_rows;
         a.ex.seq[1] = seq_s;
     }
@@ -443,7 +477,7 @@ __global__ void __launch_bounds__(kInnerThreads) inner_sparse_kernel(InnerArgs<X
                                                                       const V *val) {
     extern __shared__ double inner_lds[];
     __shared__ double sums[kInnerThreads], nw[kInnerWaves], dw[kInnerWaves], total;
-    __shared__ int group_fail;
+    __shared__ int group_fail, skip;
     const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
     const int G = gridDim.x, g = blockIdx.x, n = a.n;
     const int row0 = g * cols, nrows = max(0, min(cols, n - row0));
@@ -451,8 +485,11 @@ __global__ void __launch_bounds__(kInnerThreads) inner_sparse_kernel(InnerArgs<X
     double *xs = inner_lds;
     unsigned seq_x = inner_seq(a.ex.seq), seq_s = inner_seq(a.ex.seq + 1);
     DevScalars *ds = a.ds;
-    const InnerWait wait{a.ex.wait, &ds->inner_fail, &group_fail};
-    if (t == 0) group_fail = 0;
+    const InnerWait wait = inner_wait(a, &group_fail);
+    if (t == 0) {
+        group_fail = 0;
+        skip = G > 1 && wait.others_gave_up();
+    }
     InnerColumn<X> col;
     col.load(a, t < nrows ? (long long)row0 + t : (long long)n);
 
@@ -510,6 +547,7 @@ __global__ void __launch_bounds__(kInnerThreads) inner_sparse_kernel(InnerArgs<X
     if (val)
         for (int i = t; i < n; i += kInnerThreads) xs[i] = (double)a.x[i];
     __syncthreads();
+    if (skip) return;
     double nv = col.first(product(col.x), pre ? a.alpha0 * (ds->tol_scale * ds->tol_scale) : a.alpha0, pre);
     int it = 1;
     while (it < a.limit) {
@@ -552,6 +590,7 @@ __global__ void __launch_bounds__(kInnerThreads) inner_sparse_kernel(InnerArgs<X
     if (g == 0 && t == 0) {
         ds->bb_iter = it;
         ds->inner_total += it - 1;
+        ds->inner_counted = a.launch;
         a.ex.seq[0] = seq_x;
         a.ex.seq[1] = seq_s;
     }

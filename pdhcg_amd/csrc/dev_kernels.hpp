@@ -23,7 +23,10 @@ struct DevScalars {
     int inner_total;
     int pi_active;
     int pi_iter;
-    int inner_fail;             // a resident inner solve gave up waiting (dev_inner.hpp)
+    // resident inner solves (dev_inner.hpp), numbered from 1
+    int inner_run;      // 1 until one gives up waiting; gates what follows an inner solve
+    int inner_gave_up;  // the one that did, 0: none
+    int inner_counted;  // the last one that is in inner_total
 };
 
 template <class T> __device__ __forceinline__ T clampv(T v, T lo, T hi) { return fmax(lo, fmin(v, hi)); }
@@ -106,7 +109,9 @@ template <class X> struct EpiPrimalStep {
 // z <- w (rho z_bar + (1-rho) z) + (1-w) z0 on [x; y] (reference pdhcg_kernels.cu:283-306).
 template <class X>
 __global__ void __launch_bounds__(kBlock) halpern_kernel(const X *x0, X *x, const X *xr, const X *y0, X *y,
-                                                          const X *yr, int n, int m, double w, double rho) {
+                                                          const X *yr, int n, int m, double w, double rho,
+                                                          const int *gate) {
+    if (gate && *gate == 0) return;
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < (long long)n + m;
          i += (long long)gridDim.x * blockDim.x) {
         if (i < n) {

@@ -581,6 +581,12 @@ class SolverBase {
     virtual void graph_stats(int *windows, int *iterations) const = 0;
 };
 
+// Thrown by a read of the scalars that finds a resident inner solve given up;
+// Solver::run goes on from the state before it.
+struct InnerGaveUp : std::runtime_error {
+    InnerGaveUp() : std::runtime_error("a resident inner solve waited too long for its workgroups") {}
+};
+
 template <class V, class X> class Solver final : public SolverBase {
     template <class, class> friend class Solver;
 
@@ -633,7 +639,8 @@ template <class V, class X> class Solver final : public SolverBase {
     void read_scalars() {
         HIP_OK(hipMemcpyAsync(hs_, ds_, sizeof(DevScalars), hipMemcpyDeviceToHost, st_));
         HIP_OK(hipStreamSynchronize(st_));
-        if (hs_->inner_fail) fail("a resident inner solve waited too long for its workgroups");
+        if (hs_->inner_gave_up) throw InnerGaveUp();
+        inner_marks_.clear();
     }
     int grid(long long n) const { return blocks_for(n); }
     // one thread per element, no cap (kernels without a grid reduction)
@@ -647,6 +654,8 @@ template <class V, class X> class Solver final : public SolverBase {
     void bb_prox(double tau, bool fuse_halpern, double w);
     void init_inner_form();
     void inner_launch(double tau, bool fuse_halpern, double w);
+    int rewind_inner();
+    int run_passes(int iterations, int &done, bool at_step);
     void pdhg_step(bool fuse_halpern);
     void halpern(double w);
     void fixed_point_error();
@@ -756,6 +765,20 @@ template <class V, class X> class Solver final : public SolverBase {
     int *qrow_task_ = nullptr, *qtask_start_ = nullptr, *qci_ = nullptr;
     V *qv_ = nullptr;
     std::vector<int> row_task_;
+    // The state before each inner solve that no read of the scalars has
+    // confirmed yet, the last one being number inner_launches_
+    struct InnerMark {
+        int total_count, inner_count, host_inner;
+        X *x, *x_next;
+    };
+    std::vector<InnerMark> inner_marks_;
+    int inner_launches_ = 0;
+    int inner_give_up_at_ = 0;  // PDHCG_INNER_GIVE_UP=N: number of an inner solve that gives up (tests)
+    bool inner_gave_up_ = false;
+    // gate of the launches that change the state after an inner solve
+    const int *inner_gate() const {
+        return inner_form_ != kInnerLaunches && inner_groups_ > 1 ? &ds_->inner_run : nullptr;
+    }
     int host_inner_ = 0;  // +1 per outer iteration (reference pdhg_core_op.cu:762)
 
     // reductions and device scalars
@@ -1264,11 +1287,41 @@ template <class V, class X> void Solver<V, X>::init_inner_form() {
     int khz = 0;
     HIP_OK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
     exchange_.wait = (long long)(kInnerWaitSeconds * 1e3 * std::max(khz, 1));
+    const char *e = std::getenv("PDHCG_INNER_GIVE_UP");
+    inner_give_up_at_ = e ? std::atoi(e) : 0;
+}
+
+// Takes the loop back to the pass whose resident inner solve gave up; its
+// inner solves are launched kernel by kernel from there on.  Returns how many
+// passes before the present one that is.
+template <class V, class X> int Solver<V, X>::rewind_inner() {
+    const int first = inner_launches_ - (int)inner_marks_.size() + 1;
+    const InnerMark mark = inner_marks_.at((size_t)(hs_->inner_gave_up - first));
+    const int passes = total_count_ - mark.total_count;
+    total_count_ = mark.total_count;
+    inner_count_ = mark.inner_count;
+    host_inner_ = mark.host_inner;
+    x_ = mark.x;
+    x_next_ = mark.x_next;
+    inner_marks_.clear();
+    inner_form_ = kInnerLaunches;
+    inner_gave_up_ = true;
+    reason_ = TERMINATION_REASON_UNSPECIFIED;  // the iteration limit is noted before its evaluation reads
+    hipLaunchKernelGGL(inner_reset_kernel, dim3(1), dim3(1), 0, st_, ds_);
+    HIP_OK(hipGetLastError());
+    if (P_.verbose >= 1)
+        std::fprintf(stderr, "[inner] the workgroups of a resident inner solve did not all run at once; launch by "
+                     "launch from iteration %d\n", total_count_);
+    return passes;
 }
 
 // One inner solve in its resident form.
 template <class V, class X> void Solver<V, X>::inner_launch(double tau, bool fuse_halpern, double w) {
+    if (inner_launches_ == 0) hipLaunchKernelGGL(inner_reset_kernel, dim3(1), dim3(1), 0, st_, ds_);
+    if (inner_groups_ > 1) inner_marks_.push_back(InnerMark{total_count_, inner_count_, host_inner_, x_, x_next_});
     InnerArgs<X> a{};
+    a.launch = ++inner_launches_;
+    a.give_up = a.launch == inner_give_up_at_ ? 1 : 0;
     a.n = n_;
     a.limit = inner_limit_;
     a.halpern = fuse_halpern ? 1 : 0;
@@ -1499,9 +1552,8 @@ template <class V, class X> void Solver<V, X>::bb_prox(double tau, bool fuse_hal
         inner_launch(tau, fuse_halpern, w);
         if (fuse_halpern) std::swap(x_, x_next_);
         if (eval_) {  // the hand-over to FP64 counts inner solves that reached the limit
-            HIP_OK(hipMemcpyAsync(bb_poll_, &ds_->bb_iter, sizeof(int), hipMemcpyDeviceToHost, st_));
-            HIP_OK(hipStreamSynchronize(st_));
-            sat_run_ = (inner_limit_ > 1 && bb_poll_[0] >= inner_limit_) ? sat_run_ + 1 : 0;
+            read_scalars();
+            sat_run_ = (inner_limit_ > 1 && hs_->bb_iter >= inner_limit_) ? sat_run_ + 1 : 0;
         }
         return;
     }
@@ -1729,27 +1781,28 @@ template <class V, class X> void Solver<V, X>::pdhg_step(bool fuse_halpern) {
         bb_prox(tau, fuse_halpern, w);
     }
     host_inner_ += 1;
+    const int *gate = inner_gate();
     if (has_affine_) {
         // the dual prox point is projected onto the affine cones between the
         // SpMV and the update (reference src/pdhg_core_op.cu:809-829)
         EpiDualPrepare<X> prep{ax_, aproj_, y_, g_, cl_, cu_, sigma};
         const int t = timer_.start(kTimedDualStep, st_);
-        apply_A(xr_, prep, st_);
+        apply_A(xr_, prep, st_, gate);
         timer_.stop(kTimedDualStep, t, st_);
-        acones_.project(aproj_, aff_d_, false, nullptr, st_);
+        acones_.project(aproj_, aff_d_, false, gate, st_);
         hipLaunchKernelGGL(affine_dual_finish_kernel<X>, dim3(grid(m_)), dim3(kBlock), 0, st_, y_, yp_, yr_, ax_,
                            aproj_, sigma, store, m_);
         return;
     }
     EpiDualStep<X> depi{y_, yp_, yr_, g_, cl_, cu_, y0_, sigma, w, rho, store, fuse_halpern ? 1 : 0};
     const int t = timer_.start(kTimedDualStep, st_);
-    apply_A(xr_, depi, st_);
+    apply_A(xr_, depi, st_, gate);
     timer_.stop(kTimedDualStep, t, st_);
 }
 
 template <class V, class X> void Solver<V, X>::halpern(double w) {
     hipLaunchKernelGGL(halpern_kernel<X>, dim3(grid((long long)n_ + m_)), dim3(kBlock), 0, st_, x0_, x_, xr_, y0_, y_,
-                       yr_, n_, m_, w, P_.reflection_coefficient);
+                       yr_, n_, m_, w, P_.reflection_coefficient, inner_gate());
 }
 
 // reference src/pdhg_core_op.cu:973-1035
@@ -1897,7 +1950,7 @@ template <class V, class X> void Solver<V, X>::promote() {
             E.mdiag_ = dzeros<double>(n_);
             E.minv_ = dzeros<double>(n_);
         }
-        E.init_inner_form();
+        if (!inner_gave_up_) E.init_inner_form();
     }
     E.inner_tol_ = inner_tol_;
     E.inner_min_tol_ = inner_min_tol_;
@@ -2103,8 +2156,24 @@ template <class V, class X> void Solver<V, X>::check_termination() {
 // Main loop body, reference src/solver.cu:121-169.
 template <class V, class X> int Solver<V, X>::run(int iterations) {
     if (promoted_) return eval_->run(iterations);
+    bool at_step = false;
+    for (int done = 0;;) {
+        try {
+            const int reason = run_passes(iterations, done, at_step);
+            if (!promoted_ && !inner_marks_.empty()) read_scalars();
+            return reason;
+        } catch (const InnerGaveUp &) {
+            done -= rewind_inner();
+            at_step = true;
+        }
+    }
+}
+
+// Passes of the main loop from number `done` of `iterations`; at_step: the
+// first one has had its evaluation and restart and goes on at its step.
+template <class V, class X> int Solver<V, X>::run_passes(int iterations, int &done, bool at_step) {
     const int ef = P_.termination_evaluation_frequency;
-    for (int done = 0; done < iterations; ++done) {
+    for (; done < iterations; ++done) {
         if (reason_ != TERMINATION_REASON_UNSPECIFIED) break;
         if (!(total_count_ < P_.termination_criteria.iteration_limit)) {
             reason_ = TERMINATION_REASON_ITERATION_LIMIT;
@@ -2129,7 +2198,7 @@ template <class V, class X> int Solver<V, X>::run(int iterations) {
                              "from iteration %d\n", sat_run_, tc);
             return eval_->run(iterations - done);
         }
-        if (is_major_ || tc == 0 || tc % print_frequency(tc) == 0) {
+        if (!at_step && (is_major_ || tc == 0 || tc % print_frequency(tc) == 0)) {
             residual();
             if (!has_cones_ && !has_affine_ && is_major_ && tc < 3 * ef) infeasibility();
             cum_time_ = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start_).count();
@@ -2147,10 +2216,11 @@ template <class V, class X> int Solver<V, X>::run(int iterations) {
                 return eval_->run(iterations - done);
             }
         }
-        if (is_major_ || tc == 0) {
+        if (!at_step && (is_major_ || tc == 0)) {
             do_restart_ = should_restart();
             if (do_restart_) restart();
         }
+        at_step = false;
         is_major_ = ((tc + 1) % ef) == 0;
         const bool need_fpe = is_major_ || do_restart_;
         const double w = (double)(inner_count_ + 1) / (inner_count_ + 2);

@@ -5,7 +5,8 @@ import pytest
 import scipy.sparse as sp
 
 import pdhcg_amd
-from pdhcg_amd import PRECISION_FP64, QPData, capi, workloads
+from pdhcg_amd import PRECISION_FP64, PRECISION_MIXED, QPData, capi, workloads
+from tests.kkt import kkt
 from tests.oracle_lib import oracle_solve
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +52,63 @@ def test_one_inner_step_is_the_oracles(n, case):
     for a, b in ((g.x, o.x), (g.y, o.y)):
         error = float(np.linalg.norm(a - b) / (1.0 + np.linalg.norm(b)))
         assert error <= 1e-7
+
+
+def _low_rank(n, k, seed, affine=False):
+    rng = np.random.default_rng(seed)
+    m = max(1, n // 4)
+    A = workloads.random_sparse(rng, m, n, 4 * m)
+    x = rng.uniform(0.0, 5.0, n)
+    ax = A @ x
+    more = {}
+    if affine:
+        F = workloads.random_sparse(rng, 40, n, 160)
+        g = -F @ x
+        g[[19, 39]] += 2.0
+        more = dict(F=F, g=g, affine_cones=[(capi.CONE_STANDARD_SOC, 0, 18), (capi.CONE_STANDARD_SOC, 20, 18)])
+    return QPData(c=rng.standard_normal(n), A=A, Q=sp.diags(rng.uniform(0.8, 1.2, n)).tocsr(),
+                  R=rng.standard_normal((k, n)) / np.sqrt(n), D=rng.uniform(0.2, 0.5, k), fmt={"R": "dense"},
+                  con_lb=ax - rng.uniform(0, 1, m), con_ub=ax + rng.uniform(0, 1, m), var_lb=np.zeros(n),
+                  var_ub=np.full(n, 5.0), **more)
+
+
+_FORMS = {"rank 12, 2 workgroups": lambda: _low_rank(600, 12, 1), "rank 5, 12 workgroups": lambda: _low_rank(6000, 5, 2),
+          "rank 3, 19 workgroups": lambda: _low_rank(9300, 3, 6),
+          "affine cones": lambda: _low_rank(700, 9, 4, affine=True), "sparse, 16 workgroups": lambda: _sparse_q(1500, 0.3, 5)}
+
+
+@pytest.mark.parametrize("form", list(_FORMS))
+def test_after_a_wait_that_gives_up_the_solve_goes_on(form, monkeypatch, capfd):
+    """An inner solve whose last workgroup gives up at its first wait is
+    repeated launch by launch from the state before it: the first one, ones
+    between two reads of the scalars, one in a pass with a restart (200, 400)
+    and the last one before the iteration limit.  With three inner steps the
+    iterates do not depend on a tolerance, and the oracle with c changed in its
+    last bit moves by at most 1e-14 on these problems: 1e-9 for the other order
+    of the sums."""
+    p = _FORMS[form]()
+    kw = dict(eps=1e-14, iteration_limit=410, inner_solver_parameters=capi.inner_solver_parameters_t(3, 1e-3, 1e-9))
+    o = oracle_solve(p, **kw)
+    for launch in (0, 1, 2, 57, 200, 201, 399, 400, 410):
+        monkeypatch.setenv("PDHCG_INNER_GIVE_UP", str(launch))
+        g = pdhcg_amd.solve(p, precision=PRECISION_FP64, verbose=1, **kw)
+        note = capfd.readouterr().err
+        assert ("[inner]" in note) == (launch > 0)
+        assert launch == 0 or f"launch by launch from iteration {launch - 1}\n" in note
+        assert (g.iterations, g.inner_iterations, g.status) == (o.iterations, o.inner_iterations, o.status), launch
+        for a, b in ((g.x, o.x), (g.y, o.y)):
+            error = float(np.linalg.norm(a - b) / (1.0 + np.linalg.norm(b)))
+            assert error <= 1e-9, launch
+
+
+@pytest.mark.parametrize("precision", [PRECISION_FP64, PRECISION_MIXED])
+@pytest.mark.parametrize("form", ["rank 5, 12 workgroups", "sparse, 16 workgroups"])
+def test_whole_solve_with_a_wait_that_gives_up(form, precision, monkeypatch):
+    p = _FORMS[form]()
+    o = oracle_solve(p, eps=1e-5, iteration_limit=20000)
+    monkeypatch.setenv("PDHCG_INNER_GIVE_UP", "33")
+    g = pdhcg_amd.solve(p, precision=precision, eps=1e-5, iteration_limit=20000)
+    assert g.status == o.status == "OPTIMAL"
+    assert abs(g.pobj - o.pobj) <= 5e-5 * (1 + abs(o.pobj))
+    e = kkt(p, g.x, g.y)
+    assert max(e["rel_primal"], e["rel_dual"], e["rel_gap"]) <= 1e-4, e
