@@ -18,12 +18,19 @@
 // sequence number s + 2 only after it has read every workgroup's s + 1, and
 // those were written after their writers' last read of s.
 //
-// Residency.  A workgroup waits for the others, so all of them must be able to
-// run at once.  Small grids are launched plainly: 32 hardware queues, each with
-// such a kernel of kInnerPlainGroups (low rank: one workgroup per compute unit)
-// or kInnerSparseGroups (sparse: two per unit) workgroups, still fit the 256
-// compute units together.  Larger grids are launched cooperatively, which costs
-// about 18 us per launch more but guarantees residency.
+// Residency.  A workgroup waits for the others, so all of a grid's must be able
+// to run at once.  Each fits a compute unit of its own, and only one does in
+// places (512 threads are two waves per SIMD: 124 to 256 registers here leave
+// room for no further waiting workgroup), so grids are safe beside each other
+// while together they have at most one workgroup per unit of every XCD.
+// Workgroups are dealt to the XCDs in turn: a grid of G takes up to
+// ceil(G / 8) units of each.  Other kernels hold their units only for a time.
+// InnerResidents keeps the count for the process: while all live resident grids
+// fit the chip together they run side by side, else a launch first waits for
+// the other solvers' streams, so that they run one after the other.  Large grids
+// are launched cooperatively, which costs about 18 us per launch more: the
+// runtime then refuses a grid that would not fit the empty chip.  Grids of other
+// processes on the same GPU are in nobody's count.
 //
 // A wait that lasts kInnerWaitSeconds gives up: it notes the launch's number in
 // DevScalars and clears inner_run, and every workgroup leaves.  All that changes
@@ -34,6 +41,10 @@
 // launch (Solver::rewind_inner).
 #pragma once
 
+#include <algorithm>
+#include <mutex>
+#include <vector>
+
 #include "dev_kernels.hpp"
 
 namespace pdhcg {
@@ -42,6 +53,7 @@ constexpr int kInnerThreads = 512, kInnerWaves = kInnerThreads / kWave;
 constexpr int kInnerCols = kInnerThreads;      // columns of a workgroup, one per thread
 constexpr int kInnerColSets = kInnerCols / kWave;
 constexpr int kInnerMaxGroups = 256;           // one workgroup per compute unit
+constexpr int kInnerXcds = 8;
 constexpr int kInnerPlainGroups = 8, kInnerSparseGroups = 16;
 constexpr int kInnerAllGroups = 16;            // low rank: every workgroup sums all partial rows up to here
 constexpr int kInnerMaxRank = 80;              // rows of R: ten per wave
@@ -51,6 +63,65 @@ constexpr int kInnerSparseVars = 8192;         // x_p of the sparse form is held
 constexpr double kInnerWaitSeconds = 1.0;
 
 typedef unsigned long long xword;
+
+// The resident grids of this process: one entry per solver that has a resident
+// form of several workgroups, from its set-up to its end.
+class InnerResidents {
+  public:
+    struct Grid {
+        int device = 0, units = 0;  // units: workgroups, rounded up to a multiple of the XCDs
+        hipStream_t st = nullptr;
+        hipEvent_t ev = nullptr;    // set while the grid is counted
+        void enter() {
+            HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+            InnerResidents &all = instance();
+            std::lock_guard<std::mutex> lock(all.mu_);
+            all.live_.push_back(this);
+        }
+        // With the stream idle, or at least no resident launch in it.
+        void leave() {
+            if (!ev) return;
+            InnerResidents &all = instance();
+            std::lock_guard<std::mutex> lock(all.mu_);
+            all.live_.erase(std::remove(all.live_.begin(), all.live_.end(), this), all.live_.end());
+            (void)hipEventDestroy(ev);
+            ev = nullptr;
+        }
+        Grid() = default;
+        Grid(const Grid &) = delete;
+        Grid &operator=(const Grid &) = delete;
+        ~Grid() { leave(); }
+    };
+    static InnerResidents &instance() {
+        static InnerResidents *all = new InnerResidents;  // solvers may outlive static objects
+        return *all;
+    }
+    // Calls enqueue(), which launches g's grid, so that it runs only beside
+    // grids that fit a chip of `units` compute units with it.  Beyond that it
+    // waits on the device for all that the other solvers have enqueued (idle
+    // ones are passed over); what they launch later waits for g in turn.
+    template <class F> void launch(const Grid &g, int units, F enqueue) {
+        std::lock_guard<std::mutex> lock(mu_);
+        int total = 0;
+        for (const Grid *o : live_)
+            if (o->device == g.device) total += o->units;
+        if (total > units)
+            for (const Grid *o : live_) {
+                if (o->device != g.device || o->st == g.st) continue;
+                const hipError_t state = hipStreamQuery(o->st);
+                if (state == hipSuccess) continue;
+                if (state != hipErrorNotReady) HIP_OK(state);
+                (void)hipGetLastError();  // the query's own "not ready"
+                HIP_OK(hipEventRecord(o->ev, o->st));
+                HIP_OK(hipStreamWaitEvent(g.st, o->ev, 0));
+            }
+        enqueue();
+    }
+
+  private:
+    std::mutex mu_;
+    std::vector<Grid *> live_;
+};
 
 // Device memory of the exchanges.
 struct InnerExchange {

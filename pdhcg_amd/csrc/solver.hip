@@ -757,7 +757,8 @@ template <class V, class X> class Solver final : public SolverBase {
     // by one.
     enum InnerForm { kInnerLaunches, kInnerLowRank, kInnerSparse };
     InnerForm inner_form_ = kInnerLaunches;
-    int inner_groups_ = 0, inner_cols_ = 0;
+    int inner_groups_ = 0, inner_cols_ = 0, inner_units_ = 0;
+    InnerResidents::Grid inner_grid_;
     size_t inner_lds_ = 0;
     X *x_next_ = nullptr;  // where a resident inner solve leaves the Halpern update; then exchanged with x_
     InnerExchange exchange_ = {};
@@ -1289,6 +1290,13 @@ template <class V, class X> void Solver<V, X>::init_inner_form() {
     exchange_.wait = (long long)(kInnerWaitSeconds * 1e3 * std::max(khz, 1));
     const char *e = std::getenv("PDHCG_INNER_GIVE_UP");
     inner_give_up_at_ = e ? std::atoi(e) : 0;
+    inner_units_ = units;
+    if (inner_groups_ > 1) {
+        inner_grid_.device = dev;
+        inner_grid_.units = (inner_groups_ + kInnerXcds - 1) / kInnerXcds * kInnerXcds;
+        inner_grid_.st = st_;
+        inner_grid_.enter();
+    }
 }
 
 // Takes the loop back to the pass whose resident inner solve gave up; its
@@ -1306,6 +1314,7 @@ template <class V, class X> int Solver<V, X>::rewind_inner() {
     inner_marks_.clear();
     inner_form_ = kInnerLaunches;
     inner_gave_up_ = true;
+    inner_grid_.leave();
     reason_ = TERMINATION_REASON_UNSPECIFIED;  // the iteration limit is noted before its evaluation reads
     hipLaunchKernelGGL(inner_reset_kernel, dim3(1), dim3(1), 0, st_, ds_);
     HIP_OK(hipGetLastError());
@@ -1344,33 +1353,38 @@ template <class V, class X> void Solver<V, X>::inner_launch(double tau, bool fus
     a.m_diag = precond_ ? mdiag_ : nullptr;
     a.ex = exchange_;
     a.ds = ds_;
-    if (inner_form_ == kInnerSparse) {
-        hipLaunchKernelGGL((inner_sparse_kernel<V, X, Acc>), dim3(inner_groups_), dim3(kInnerThreads),
-                           inner_lds_, st_, a, inner_cols_, (const int *)qrow_task_, (const int *)qtask_start_,
-                           (const int *)qci_, (const V *)qv_);
-        HIP_OK(hipGetLastError());
-        return;
-    }
-    auto go = [&](auto kernel) {
-        const V *R = Rd_;
-        const double *dd = ddiag_, *de = ddense_;
-        void *args[] = {&a, &R, &k_, &dd, &de, &dkind_};
-        if (inner_groups_ > kInnerPlainGroups)
-            HIP_OK(hipLaunchCooperativeKernel((const void *)kernel, dim3(inner_groups_), dim3(kInnerThreads), args, 0,
-                                              st_));
-        else
-            HIP_OK(hipLaunchKernel((const void *)kernel, dim3(inner_groups_), dim3(kInnerThreads), args, 0, st_));
+    auto enqueue = [&]() {
+        if (inner_form_ == kInnerSparse) {
+            hipLaunchKernelGGL((inner_sparse_kernel<V, X, Acc>), dim3(inner_groups_), dim3(kInnerThreads), inner_lds_,
+                               st_, a, inner_cols_, (const int *)qrow_task_, (const int *)qtask_start_,
+                               (const int *)qci_, (const V *)qv_);
+            HIP_OK(hipGetLastError());
+            return;
+        }
+        auto go = [&](auto kernel) {
+            const V *R = Rd_;
+            const double *dd = ddiag_, *de = ddense_;
+            void *args[] = {&a, &R, &k_, &dd, &de, &dkind_};
+            if (inner_groups_ > kInnerPlainGroups)
+                HIP_OK(hipLaunchCooperativeKernel((const void *)kernel, dim3(inner_groups_), dim3(kInnerThreads), args,
+                                                  0, st_));
+            else
+                HIP_OK(hipLaunchKernel((const void *)kernel, dim3(inner_groups_), dim3(kInnerThreads), args, 0, st_));
+        };
+        // rows of R per wave
+        if (k_ <= 8) go(inner_lowrank_kernel<V, X, 1>);
+        else if (k_ <= 16) go(inner_lowrank_kernel<V, X, 2>);
+        else if (k_ <= 32) go(inner_lowrank_kernel<V, X, 4>);
+        else if (k_ <= 56) go(inner_lowrank_kernel<V, X, 7>);
+        else go(inner_lowrank_kernel<V, X, 10>);
     };
-    // rows of R per wave
-    if (k_ <= 8) go(inner_lowrank_kernel<V, X, 1>);
-    else if (k_ <= 16) go(inner_lowrank_kernel<V, X, 2>);
-    else if (k_ <= 32) go(inner_lowrank_kernel<V, X, 4>);
-    else if (k_ <= 56) go(inner_lowrank_kernel<V, X, 7>);
-    else go(inner_lowrank_kernel<V, X, 10>);
+    if (inner_grid_.ev) InnerResidents::instance().launch(inner_grid_, inner_units_, enqueue);
+    else enqueue();
 }
 
 template <class V, class X> Solver<V, X>::~Solver() {
     if (st_) (void)hipStreamSynchronize(st_);
+    inner_grid_.leave();
     delete eval_;
     for (GraphWindow &g : graphs_) release_graph(g);
     if (dyn_) (void)hipFree(dyn_);

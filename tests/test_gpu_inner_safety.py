@@ -1,5 +1,7 @@
 """The resident inner solve (dev_inner.hpp) where nothing but its own rules
 keeps workgroups from each other's data."""
+from threading import Barrier, Thread
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -112,3 +114,70 @@ def test_whole_solve_with_a_wait_that_gives_up(form, precision, monkeypatch):
     assert abs(g.pobj - o.pobj) <= 5e-5 * (1 + abs(o.pobj))
     e = kkt(p, g.x, g.y)
     assert max(e["rel_primal"], e["rel_dual"], e["rel_gap"]) <= 1e-4, e
+
+
+def test_solves_beside_each_other_wait_for_room(monkeypatch, capfd):
+    """Three solvers stepped from three threads at once, whose resident
+    workgroups (200, 144 and 16 compute units) do not fit the chip together:
+    none of them gives up a wait, and each goes the way it goes alone, bit for
+    bit."""
+    monkeypatch.setenv("PDHCG_SPMV_SHIFT", "0")  # otherwise picked by timing
+    problems = [_low_rank(100000, 6, 11), _low_rank(70000, 20, 12), _sparse_q(1500, 0.3, 13)]
+    count = [1500, 1500, 3000]
+
+    def stepper(i):
+        return pdhcg_amd.Stepper(problems[i], eps=1e-15, iteration_limit=10 ** 6, verbose=1)
+
+    alone = []
+    for i in range(3):
+        s = stepper(i)
+        s.run(count[i])
+        alone.append(s.result())
+        s.close()
+    steppers = [stepper(i) for i in range(3)]
+    gate = Barrier(3)
+
+    def step(i):
+        gate.wait()
+        for _ in range(10):
+            steppers[i].run(count[i] // 10)
+
+    threads = [Thread(target=step, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, s in zip(alone, steppers):
+        b = s.result()
+        s.close()
+        assert (a.iterations, a.inner_iterations) == (b.iterations, b.inner_iterations)
+        assert a.status == "UNSPECIFIED"  # all the passes asked for
+        assert np.array_equal(a.x, b.x) and np.array_equal(a.y, b.y)
+    assert "[inner]" not in capfd.readouterr().err
+
+
+def test_solvers_of_one_thread_in_turn(monkeypatch):
+    """Two solvers alive at once, each of more than half the chip, stepped in
+    turn: each goes the way it goes alone."""
+    monkeypatch.setenv("PDHCG_SPMV_SHIFT", "0")
+    problems = [_low_rank(80000, 4, 21), _low_rank(90000, 4, 22)]
+
+    def finish(s):
+        r = s.result()
+        s.close()
+        return r
+
+    alone = []
+    for p in problems:
+        s = pdhcg_amd.Stepper(p)
+        for _ in range(6):
+            s.run(7)
+        alone.append(finish(s))
+    both = [pdhcg_amd.Stepper(p) for p in problems]
+    for _ in range(6):
+        for s in both:
+            s.run(7)
+    for a, s in zip(alone, both):
+        b = finish(s)
+        assert a.iterations == b.iterations == 42
+        assert np.array_equal(a.x, b.x) and np.array_equal(a.y, b.y)
