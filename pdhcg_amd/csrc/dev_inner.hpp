@@ -334,8 +334,9 @@ template <class X> struct InnerColumn {
 // to kInnerMaxRank.
 //
 // Workgroup g owns kInnerCols columns and keeps its slice of R in registers
-// for the whole inner solve (up to 160 of a thread's 256 at rank 80 in FP64),
-// so that R is read once per outer iteration instead of twice per body: wave w
+// for the whole inner solve (at ranks 57 to 80 in FP64 160 of a thread's 256
+// registers, of which 13 other values are spilled, in FP32 as well: 56 bytes of
+// scratch per lane; no spills up to rank 56), so that R is read once per outer iteration instead of twice per body: wave w
 // holds rows w, w + 8, ... and lane l of it columns l, l + 64, ...  R x is
 // then a sum over a lane's eight columns and a butterfly over the wave, with
 // no sum across waves; R'u is a sum over a thread's rows and, through LDS, the

@@ -1237,7 +1237,12 @@ template <class V, class X> void Solver<V, X>::init_inner(const ScaledProblem &s
 // iterations (milliseconds in the iteration): n = 600, rank 50: 80 -> 18;
 // n = 4000, rank 50: 136 -> 26; n = 20 000, rank 30: 99 -> 37; n = 100 000,
 // rank 50: 147 -> 52; n = 130 000, rank 50: 163 -> 56; sparse Q of 2000
-// variables (41 entries per row): 15-23 -> 5.5 us per body.
+// variables (41 entries per row): 15-23 -> 5.5 us per body.  Ranks 57 to 80,
+// whose kernel spills a few registers, and FP32, per 300 outer iterations with
+// the same number of bodies (FP64; mixed precision): n = 600, rank 57 68 -> 18;
+// 68 -> 23, rank 80 72 -> 19; 76 -> 25; n = 20 000, rank 57 87 -> 28; 85 -> 33;
+// n = 100 000, rank 64 92 -> 30; 83 -> 37, rank 80 92 -> 31; 81 -> 38 (rank 56
+// 90 -> 31; 86 -> 38).
 template <class V, class X> void Solver<V, X>::init_inner_form() {
     if (!bb_ || has_cones_ || n_ <= 0) return;
     const bool plus = qtype_ == PDHCG_LOW_RANK_PLUS_SPARSE_Q;

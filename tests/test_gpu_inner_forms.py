@@ -9,7 +9,7 @@ import pytest
 import scipy.sparse as sp
 
 import pdhcg_amd
-from pdhcg_amd import PRECISION_FP64, PRECISION_MIXED, QPData, workloads
+from pdhcg_amd import PRECISION_FP64, PRECISION_MIXED, QPData, capi, workloads
 from tests.kkt import kkt
 from tests.oracle_lib import oracle_solve
 
@@ -64,3 +64,33 @@ def test_sparse_q(n, per_row, precision):
     S = (S + S.T).tocsr()
     Q = (S * (0.5 / max(1.0, abs(S).sum(axis=1).max())) + sp.diags(rng.uniform(0.6, 1.5, n))).tocsr()
     _check(_rows(rng, n, max(1, n // 4), Q=Q), precision)
+
+
+# 65 workgroups (a lane sums more than one of a row's), all 256 of the chip, and
+# the launched form above them
+@pytest.mark.parametrize("n,k", [(33000, 80), (131072, 50), (131073, 50)])
+def test_low_rank_large_grids(n, k):
+    """The oracle's iterates after 16 iterations of three inner steps each.
+    With c changed in its last bit the oracle moves by 2e-15 there; the sums of
+    up to 131 073 terms in another order are off by at most 1e5 such bits."""
+    rng = np.random.default_rng(n)
+    p = _rows(rng, n, n // 4, Q=sp.diags(rng.uniform(0.8, 1.2, n)).tocsr(),
+              R=rng.standard_normal((k, n)) / np.sqrt(n), D=rng.uniform(0.2, 0.5, k), fmt={"R": "dense"})
+    kw = dict(eps=1e-14, iteration_limit=16, inner_solver_parameters=capi.inner_solver_parameters_t(3, 1e-3, 1e-9))
+    o = oracle_solve(p, **kw)
+    g = pdhcg_amd.solve(p, precision=PRECISION_FP64, **kw)
+    assert (g.iterations, g.inner_iterations) == (o.iterations, o.inner_iterations)
+    for a, b in ((g.x, o.x), (g.y, o.y)):
+        error = float(np.linalg.norm(a - b) / (1.0 + np.linalg.norm(b)))
+        assert error <= 1e-10
+
+
+@pytest.mark.parametrize("n,k", [(33000, 80), (131072, 50)])
+def test_low_rank_large_grids_mixed(n, k):
+    rng = np.random.default_rng(n)
+    p = _rows(rng, n, n // 4, Q=sp.diags(rng.uniform(0.8, 1.2, n)).tocsr(),
+              R=rng.standard_normal((k, n)) / np.sqrt(n), D=rng.uniform(0.2, 0.5, k), fmt={"R": "dense"})
+    g = pdhcg_amd.solve(p, precision=PRECISION_MIXED, eps=1e-4, iteration_limit=20000)
+    assert g.status == "OPTIMAL"
+    e = kkt(p, g.x, g.y)
+    assert max(e["rel_primal"], e["rel_dual"], e["rel_gap"]) <= 1e-3, e
