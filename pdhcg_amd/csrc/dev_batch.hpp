@@ -359,13 +359,14 @@ template <class T, int BT> struct Ctx {
     }
 
     // Sums of U rows of R times x over the wave; the lanes take pairs of
-    // columns, four per row in flight.  row(a, i), x(i): the pair at column i.
+    // columns, four per row in flight, in four sums each (in FP32 a sum's length
+    // is its error bound).  row(a, i), x(i): the pair at column i.
     template <int U, class Row, class Vec> __device__ __forceinline__ void row_sums(Row row, Vec x, double (&out)[U]) const {
         typedef typename Pair<T>::type P2;
         const int half = I.pn / 2, lane = threadIdx.x % kWave;
-        T s[U][2];
+        T s[U][4];
 #pragma unroll
-        for (int a = 0; a < U; ++a) s[a][0] = s[a][1] = T(0);
+        for (int a = 0; a < U; ++a) s[a][0] = s[a][1] = s[a][2] = s[a][3] = T(0);
         for (int p = lane; p < half; p += 4 * kWave) {
             P2 v[U][4], xv[4];
 #pragma unroll
@@ -383,12 +384,13 @@ template <class T, int BT> struct Ctx {
             for (int q = 0; q < 4; ++q)
 #pragma unroll
                 for (int a = 0; a < U; ++a) {
-                    s[a][0] += v[a][q][0] * xv[q][0];
-                    s[a][1] += v[a][q][1] * xv[q][1];
+                    s[a][2 * (q & 1)] += v[a][q][0] * xv[q][0];
+                    s[a][2 * (q & 1) + 1] += v[a][q][1] * xv[q][1];
                 }
         }
 #pragma unroll
-        for (int a = 0; a < U; ++a) out[a] = wave_total((double)s[a][0] + (double)s[a][1]);
+        for (int a = 0; a < U; ++a)
+            out[a] = wave_total(((double)s[a][0] + (double)s[a][1]) + ((double)s[a][2] + (double)s[a][3]));
     }
     // put(r, row r of M times x) in lane 0, for the rows [0, k) of a dense
     // k x pn M whose first `res` rows are the resident ones in LDS; x(i) as in
@@ -447,15 +449,15 @@ template <class T, int BT> struct Ctx {
     __device__ __forceinline__ void low_rank_columns(int p, T (&out)[2]) const {
         columns(R, I.k, resident, lds_u(), p, out);
     }
-    // Columns 2 p and 2 p + 1 of M'u for the M of all_rows and u in LDS.  The
-    // first eight rows outside LDS are in flight while the resident ones are
-    // added.
+    // Columns 2 p and 2 p + 1 of M'u for the M of all_rows and u in LDS, each in
+    // four sums.  The first eight rows outside LDS are in flight while the
+    // resident ones are added.
     __device__ __forceinline__ void columns(const T *M, int k, int resident, const double *u, int p, T (&out)[2]) const {
         typedef typename Pair<T>::type P2;
         constexpr int U = 8;
         const int pn = I.pn, lcol = room + 2 * p;
         const T *col = M + 2 * p;
-        T s0 = T(0), s1 = T(0);
+        T s[4][2] = {};
         int r = resident;
         P2 g[U];
 #pragma unroll
@@ -473,8 +475,8 @@ template <class T, int BT> struct Ctx {
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
                 const T uj = j + a < resident ? (T)u[j + a] : T(0);
-                s0 += v[a][0] * uj;
-                s1 += v[a][1] * uj;
+                s[a][0] += v[a][0] * uj;
+                s[a][1] += v[a][1] * uj;
             }
         }
         while (r < k) {
@@ -487,15 +489,15 @@ template <class T, int BT> struct Ctx {
 #pragma unroll
             for (int a = 0; a < U; ++a) {
                 const T uj = r + a < k ? (T)u[r + a] : T(0);
-                s0 += g[a][0] * uj;
-                s1 += g[a][1] * uj;
+                s[a % 4][0] += g[a][0] * uj;
+                s[a % 4][1] += g[a][1] * uj;
             }
 #pragma unroll
             for (int a = 0; a < U; ++a) g[a] = nx[a];
             r += U;
         }
-        out[0] = s0;
-        out[1] = s1;
+        out[0] = (s[0][0] + s[1][0]) + (s[2][0] + s[3][0]);
+        out[1] = (s[0][1] + s[1][1]) + (s[2][1] + s[3][1]);
     }
     // Copies x into LDS (when the product's vector is staged); a barrier must follow.
     __device__ __forceinline__ void stage(const T *x) const {
