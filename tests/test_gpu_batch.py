@@ -8,6 +8,8 @@ solve tolerance for problems without affine cones, and for the portfolios
 the budget row and the tracking-error limit.  Problems outside the batch's
 scope come back as None while the rest of the batch is solved.
 """
+from dataclasses import replace
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -140,17 +142,26 @@ def test_batch_thread_counts_match_oracle(threads, monkeypatch):
             _agree(p, g, oracle_solve(p, eps=EPS, iteration_limit=200000), affine=i >= len(cases))
 
 
-@pytest.mark.parametrize("rows", ["4", "16", "64"])
-def test_batch_row_forms_match_oracle(rows, monkeypatch):
-    # the three row-length thresholds the launch probe chooses between
-    # (a wavefront or a thread per row of A and A'), pinned, to the same bar;
-    # rows of 8 to 32 entries on average make each threshold split differently
-    monkeypatch.setenv("PDHCG_BATCH_ROWS", rows)
-    cases = [("lp", 120, 3), ("diag", 150, 4), ("lowrank_diag", 160, 5)]
-    problems = [workloads.random_problem(kind, seed=seed, n=n, m=max(10, n // 3)) for kind, n, seed in cases]
+@pytest.mark.parametrize("fill", [0.1, 0.33, 0.34, 0.9])
+def test_batch_row_forms_match_oracle(fill):
+    # A on both sides of the rule for its dense form (3 nnz >= m n): streamed
+    # in chunks with its transpose, and stored dense without one; the
+    # portfolios' factor rows are mostly full
+    problems = []
+    for i, (kind, n, seed) in enumerate([("lp", 120, 3), ("diag", 150, 4), ("lowrank_diag", 160, 5)]):
+        p = workloads.random_problem(kind, seed=seed, n=n, m=max(10, n // 3))
+        rng = np.random.default_rng((seed, i))
+        m, n = p.A.shape
+        ones = np.zeros(m * n, dtype=bool)
+        ones[rng.permutation(m * n)[: int(round(fill * m * n))]] = True
+        A = sp.csr_matrix(np.where(ones.reshape(m, n), rng.standard_normal((m, n)), 0.0))
+        assert (3 * A.nnz >= m * n) == (fill > 1 / 3)
+        ax = A @ rng.uniform(-1.0, 1.0, n)
+        problems.append(replace(p, A=A, con_lb=ax - rng.uniform(0, 1, m), con_ub=ax + rng.uniform(0, 1, m)))
+    cases = len(problems)
     problems += workloads.portfolio_batch(2, seed=17, n_range=(60, 150), k_range=(10, 40))
     for precision in (pdhcg_amd.PRECISION_FP64, PRECISION_MIXED):
         sols = pdhcg_amd.solve_batch(problems, precision=precision, eps=EPS, iteration_limit=200000,
                                      time_limit=60.0)
         for i, (p, g) in enumerate(zip(problems, sols)):
-            _agree(p, g, oracle_solve(p, eps=EPS, iteration_limit=200000), affine=i >= len(cases))
+            _agree(p, g, oracle_solve(p, eps=EPS, iteration_limit=200000), affine=i >= cases)

@@ -1,14 +1,16 @@
-"""The round-robin schedule of the PSD projection's register-resident
-eigenvector rows (psd_project_kernel in pdhcg_amd/csrc/dev_cones.hpp).
+"""The round-robin schedule of the PSD projection by position
+(psd_positions_kernel in pdhcg_amd/csrc/dev_cones.hpp, orders 2 to 128).
 
-Lane L holds the rows (up[L], dn[L]) of pair L.  After each round the up rows
-move one lane right, the down rows one lane left, lane 0 keeps its up row,
-lane 1 takes lane 0's down row and the last lane takes its own up row (a
-single pair stays in place).  This restates those moves and checks the
-properties the Jacobi sweep relies on: every round pairs all kp indices
-disjointly, every pair of indices meets exactly once in kp - 1 rounds, and the
-positions are back at their start after a sweep.  (The rotations themselves
-are checked against the oracle by the GPU PSD tests at orders 97..128.)
+Position L holds an up and a down element, which a round rotates against each
+other.  After each round the up elements move one position right, the down
+elements one position left, position 0 keeps its up element, position 1 takes
+position 0's down element and the last position's up element becomes its down
+element (a single pair stays in place); the blocks of the matrix and the rows of
+V' are written to where their elements stand next.  This restates those moves
+and checks the properties the Jacobi sweep relies on: every round pairs all kp
+elements disjointly, every pair meets exactly once in kp - 1 rounds, and the
+elements are back at their places after a sweep.  (The rotations themselves are
+checked by the GPU PSD tests.)
 """
 import itertools
 
