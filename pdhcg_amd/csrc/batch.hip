@@ -55,7 +55,7 @@ __global__ void narrow_kernel(const double *a, float *b, long long n) {
 // Jacobi diagonal, g, row bounds) keep their FP64 values.
 __global__ void widen_iterates_kernel(const Inst *insts, const float *s32, double *s64) {
     const Inst I = insts[blockIdx.x];
-    const int nv[] = {vX0, vX, vXP, vXR, vATY, vDS, vGR, vDIR, vQX, vPB, vDX, vMD, vMI};
+    const int nv[] = {vX0, vX, vXP, vXR, vATY, vDS, vGR, vDIR, vQX, vDX, vMD, vMI};
     const int mv[] = {wY0, wY, wYP, wYR, wAX, wDY, wPRES, wPSL, wAPR, wAMEM};
     for (int w : nv)
         for (int i = threadIdx.x; i < I.n; i += blockDim.x) {
@@ -124,7 +124,7 @@ struct Packed {
     std::vector<int> ai;     // A rp, A ci, At rp, At ci
     std::vector<double> av;  // A v, At v, R dense, D
     std::vector<double> slab;   // n- and m-vectors
-    std::vector<double> wslab;  // k-vectors and per-cone values
+    std::vector<double> wslab;  // per-cone values
     std::vector<Cone> cones;
     HostState st;
 };
@@ -290,7 +290,7 @@ bool pack(const qp_problem_t *prob, const pdhg_parameters_t &P, Packed &k, const
     I.pw0 = P.bound_objective_rescaling ? 1.0 : (sp.obj_norm + 1.0) / (sp.bound_norm + 1.0);
     // the slab (FP64), starting point projected onto the box
     k.slab.assign((size_t)slab_size(n, m), 0.0);
-    k.wslab.assign((size_t)wslab_size(I.k, I.ncones), 0.0);
+    k.wslab.assign((size_t)wslab_size(I.ncones), 0.0);
     auto N = [&](int w) { return k.slab.data() + (size_t)w * I.pn; };
     auto M = [&](int w) { return k.slab.data() + (size_t)kNVec * I.pn + (size_t)w * I.pm; };
     for (int i = 0; i < n; ++i) {
@@ -485,7 +485,7 @@ extern "C" int pdhcg_solve_batch(const qp_problem_t *const *problems, int count,
             const long long nnz = I.a_nnz;
             bool ok = I.rdense % 4 == 0 && I.vec % 4 == 0 && I.dmat >= I.rdense + (long long)I.k * I.pn &&
                       I.dmat <= voff[b + 1] && I.vec + slab_size(I.n, I.m) <= soff[b + 1] &&
-                      I.wvec + wslab_size(I.k, I.ncones) <= woff[b + 1] && I.cone0 + I.ncones <= coff[b + 1];
+                      I.wvec + wslab_size(I.ncones) <= woff[b + 1] && I.cone0 + I.ncones <= coff[b + 1];
             if (I.a_dense) {
                 ok = ok && I.m <= kMaxRank && I.a_v % 4 == 0 && I.rdense >= I.a_v + (long long)I.m * I.pn;
             } else {

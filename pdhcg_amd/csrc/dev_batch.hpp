@@ -68,7 +68,7 @@ struct Inst {
     int a_nnz, a_chunk, at_chunk;  // entries of A; int-pool offsets of the products' chunk tables
     long long a_v, at_v;           // value-pool offsets of the matrix values
     long long vec;                 // slab offset of the problem's n- and m-vectors
-    long long wvec;                // FP64 slab offset of its k-vectors and per-cone values
+    long long wvec;                // FP64 slab offset of its per-cone values
     long long rdense, dmat;        // value-pool offsets of R (k x pn row-major, zero padded) and D
     double cbr, ovr, obj_const, obj_norm, bound_norm, step, pw0, nonconvexity;
 };
@@ -86,18 +86,17 @@ struct Out {
 };
 
 // Slab layout: n-vectors, then m-vectors (storage type of the kernel); the
-// FP64 slab: k-vectors, then per-cone values.
-enum NVec { vC, vLB, vUB, vVR, vQD, vDH, vX0, vX, vXP, vXR, vATY, vDS, vGR, vDIR, vQX, vPB, vDX, vMD, vMI, vLBF, vUBF,
+// FP64 slab: per-cone values.  (The k-vectors live in LDS.)
+enum NVec { vC, vLB, vUB, vVR, vQD, vDH, vX0, vX, vXP, vXR, vATY, vDS, vGR, vDIR, vQX, vDX, vMD, vMI, vLBF, vUBF,
             kNVec };
 enum MVec { wG, wCL, wCU, wCLF, wCUF, wCR, wY0, wY, wYP, wYR, wAX, wDY, wPRES, wPSL, wAPR, wAMEM, wAFD, kMVec };
-constexpr int kKVec = 0;      // the k-vectors live in LDS
 constexpr int kConeVals = 3;  // projection warm start, residual warm start, complementarity
 
 __host__ __device__ inline int padded4(int n) { return (n + 3) & ~3; }
 inline long long slab_size(int n, int m) {
     return (long long)kNVec * padded4(n) + (long long)kMVec * padded4(m);
 }
-inline long long wslab_size(int k, int ncones) { return (long long)kKVec * k + (long long)kConeVals * ncones; }
+inline long long wslab_size(int ncones) { return (long long)kConeVals * ncones; }
 
 // Chunks of kChunk entries in which a product streams its matrix, at least one.
 constexpr int kChunk = 4096;
@@ -328,7 +327,7 @@ template <class T, int BT> struct Ctx {
     int stage_room, room, resident;
     __device__ T *nv(int which) const { return V + (long long)which * I.pn; }
     __device__ T *mv(int which) const { return V + (long long)kNVec * I.pn + (long long)which * I.pm; }
-    __device__ double *cv(int which) const { return W + (long long)kKVec * I.k + (long long)which * I.ncones; }
+    __device__ double *cv(int which) const { return W + (long long)which * I.ncones; }
     // Products with A and A'.  A dense A (factor models: a few full rows) is
     // read once per product without indices, by the passes of a dense R.
     __device__ void A(const T *x, T *y) const {
