@@ -2,7 +2,7 @@
 // as one launch per outer iteration, for problems that fit the chip: its first
 // step, every loop body, the reflection and the Halpern update.
 //
-// Launched kernel by kernel, a body is six launches (four for a sparse Q) of
+// Launched kernel by kernel, a body is six launches (five for a sparse Q) of
 // 2-4 us each whatever the problem's size: 26 us per body at n = 60, 11-23 us
 // with a 2000-variable sparse Q.  Here the columns are split over at most
 // kInnerMaxGroups workgroups that stay resident, and a body costs two
