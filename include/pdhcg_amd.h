@@ -8,8 +8,9 @@
  *
  * The precision and graph-window switches are process-wide and unsynchronised:
  * set them before solves start, not while another thread is solving.  Each
- * solve owns its HIP stream and device buffers; a cancel request applies to
- * every running solve.
+ * solve owns its HIP stream and device buffers; solves whose resident inner
+ * solves do not fit the device together take turns on it.  A cancel request
+ * applies to every running solve.
  */
 #pragma once
 
