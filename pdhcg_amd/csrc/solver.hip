@@ -2002,6 +2002,7 @@ template <class V, class X> void Solver<V, X>::promote() {
     E.host_inner_ = host_inner_ + hs_->inner_total;
     E.graph_on_ = false;
     HIP_OK(hipStreamSynchronize(st_));
+    inner_grid_.leave();
     promoted_ = true;
 }
 
